@@ -29,6 +29,7 @@
 #include "awcpml.h"
 #include "launch.h"
 #include "stencil_kernels.h"
+#include "transfer_kernels.h"
 
 using awcpml::StencilArgs;
 
@@ -137,6 +138,11 @@ struct awcpml_plan {
     int64_t it = 0;   // steps done
     int rot = 0;      // p[rot] = pold, p[rot+1] = pcur, p[rot+2] = pnew
     int par = 0;      // psi[..][par] = previous step
+
+    // dense FP64 rows on their way to or from the host (transfer_kernels.h),
+    // allocated on first use
+    double* stage = nullptr;
+    int64_t stage_elems = 0;
 
     hipStream_t stream = nullptr;
     // captured step sequences (hipGraph), keyed by first step and length
@@ -247,11 +253,128 @@ void dfree(void*& ptr) {
     ptr = nullptr;
 }
 
-// host FP64 values -> device buffer of the plan's precision
+// Staged transfers take at most this many FP64 values at a time (32 MiB per
+// plan; longer arrays go in pieces, in order on the plan's stream).
+constexpr int64_t kStageElems = 4ll << 20;
+// Unpadded FP32 values up to this many (a shot's traces) are copied as they
+// are and converted by the host: the launch and the doubled copy of the
+// device's way cost more (57,600 values: 19 us more).
+constexpr int64_t kHostConvert = 256ll << 10;
+
+// The plan's staging buffer, of at least `row` and preferably `want` elements.
+int stage_buffer(awcpml_plan* P, int64_t row, int64_t want) {
+    want = std::max(row, std::min(want, kStageElems));
+    if (P->stage_elems >= want) return AWCPML_OK;
+    if (P->stage) {
+        HIP_TRY(hipStreamSynchronize(P->stream));
+        (void)hipFree(P->stage);
+        P->stage = nullptr;
+        P->stage_elems = 0;
+    }
+    for (int64_t n = want;; n = std::max(row, n / 8)) {
+        void* v = nullptr;
+        const int st = dalloc(&v, (size_t)n * 8);
+        if (!st) {
+            P->stage = (double*)v;
+            P->stage_elems = n;
+            return AWCPML_OK;
+        }
+        if (st != AWCPML_ERR_NOMEM || n <= row) return st;
+        (void)hipGetLastError();  // a smaller piece may still fit
+    }
+}
+
+// How a transfer of `rows` rows of nx values (device pitch px) is cut: rows
+// as they are, or, where they lie back to back, runs of kRowSeg values (so
+// that a long unpadded array goes through the stage in pieces too).
+struct RowPieces {
+    int64_t row, pitch, rows;
+    bool flat;
+    RowPieces(int64_t nx, int64_t px, int64_t nrows) : row(nx), pitch(px), rows(nrows) {
+        flat = px == nx;
+        if (flat) {
+            row = pitch = awcpml::kRowSeg;
+            rows = (nx * nrows + row - 1) / row;
+        }
+    }
+    // convert n pieces holding len values in all
+    template <typename S, typename D>
+    void convert(awcpml_plan* P, const S* src, int64_t spitch, D* dst, int64_t dpitch, int64_t n,
+                 int64_t len) const {
+        const int64_t nx = flat ? len : row, nr = flat ? 1 : n;
+        const int64_t blocks = (nx + awcpml::kRowSeg - 1) / awcpml::kRowSeg * nr;
+        awcpml::convert_rows<S, D><<<dim3((unsigned)std::min<int64_t>(blocks, 8192)), dim3(256), 0, P->stream>>>(
+            src, dst, nx, spitch, dpitch, nr);
+    }
+};
+
+// Dense host rows of nx FP64 values -> device rows of pitch px in T.
+template <typename T>
+int upload_rows_t(awcpml_plan* P, T* dst, const double* src, int64_t nx, int64_t px, int64_t rows) {
+    if (nx == 0 || rows == 0) return AWCPML_OK;
+    if (sizeof(T) == 8 && px == nx) {
+        HIP_TRY(hipMemcpyAsync(dst, src, (size_t)(nx * rows) * 8, hipMemcpyHostToDevice, P->stream));
+        return AWCPML_OK;
+    }
+    const RowPieces R(nx, px, rows);
+    int st = stage_buffer(P, R.row, nx * rows);
+    if (st) return st;
+    const int64_t step = P->stage_elems / R.row;
+    for (int64_t r = 0; r < R.rows; r += step) {
+        const int64_t n = std::min(step, R.rows - r), len = std::min(n * R.row, nx * rows - r * R.row);
+        HIP_TRY(hipMemcpyAsync(P->stage, src + r * R.row, (size_t)len * 8, hipMemcpyHostToDevice, P->stream));
+        R.convert(P, (const double*)P->stage, R.row, dst + r * R.pitch, R.pitch, n, len);
+        HIP_TRY(hipGetLastError());
+    }
+    return AWCPML_OK;
+}
+
+// Device rows of pitch px in T -> dense host rows of nx FP64 values;
+// returns with the values in place.
+template <typename T>
+int download_rows_t(awcpml_plan* P, double* dst, const T* src, int64_t nx, int64_t px, int64_t rows) {
+    if (nx == 0 || rows == 0) return AWCPML_OK;
+    if (sizeof(T) == 8 && px == nx) {
+        HIP_TRY(hipMemcpyAsync(dst, src, (size_t)(nx * rows) * 8, hipMemcpyDeviceToHost, P->stream));
+        HIP_TRY(hipStreamSynchronize(P->stream));
+        return AWCPML_OK;
+    }
+    const int64_t count = nx * rows;
+    if (sizeof(T) == 4 && px == nx && count <= kHostConvert) {
+        std::vector<T> tmp((size_t)count);
+        HIP_TRY(hipMemcpyAsync(tmp.data(), src, (size_t)count * sizeof(T), hipMemcpyDeviceToHost, P->stream));
+        HIP_TRY(hipStreamSynchronize(P->stream));
+        for (int64_t q = 0; q < count; ++q) dst[q] = (double)tmp[(size_t)q];
+        return AWCPML_OK;
+    }
+    const RowPieces R(nx, px, rows);
+    int st = stage_buffer(P, R.row, nx * rows);
+    if (st) return st;
+    const int64_t step = P->stage_elems / R.row;
+    for (int64_t r = 0; r < R.rows; r += step) {
+        const int64_t n = std::min(step, R.rows - r), len = std::min(n * R.row, nx * rows - r * R.row);
+        R.convert(P, src + r * R.pitch, R.pitch, P->stage, R.row, n, len);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(dst + r * R.row, P->stage, (size_t)len * 8, hipMemcpyDeviceToHost, P->stream));
+    }
+    HIP_TRY(hipStreamSynchronize(P->stream));
+    return AWCPML_OK;
+}
+
+int download_rows(awcpml_plan* P, double* dst, const void* src, int64_t nx, int64_t px, int64_t rows) {
+    return P->dtype == AWCPML_F64 ? download_rows_t<double>(P, dst, (const double*)src, nx, px, rows)
+                                  : download_rows_t<float>(P, dst, (const float*)src, nx, px, rows);
+}
+
+// host FP64 values -> device buffer of the plan's precision.  Short FP32
+// vectors (coefficients) are rounded on the host; from 16 Ki values on the
+// device's conversion is the shorter way (both round to nearest even).
 int upload(awcpml_plan* P, void* dst, const double* src, size_t count) {
     if (count == 0) return AWCPML_OK;
     if (P->dtype == AWCPML_F64) {
         HIP_TRY(hipMemcpyAsync(dst, src, count * 8, hipMemcpyHostToDevice, P->stream));
+    } else if (count >= (16u << 10)) {
+        return upload_rows_t<float>(P, (float*)dst, src, (int64_t)count, (int64_t)count, 1);
     } else {
         std::vector<float> tmp(count);
         for (size_t i = 0; i < count; ++i) tmp[i] = (float)src[i];
@@ -1338,6 +1461,7 @@ int awcpml_plan_destroy(awcpml_plan* P) {
     dfree(P->d_rec_start);
     dfree(P->d_traces);
     dfree(P->ck);
+    if (P->stage) (void)hipFree(P->stage);
     if (P->stream) (void)hipStreamDestroy(P->stream);
     delete P;
     return AWCPML_OK;
@@ -1354,35 +1478,18 @@ int awcpml_set_model(awcpml_plan* P, const double* fact, const double* inv_d, co
         P->inv_d2[a] = inv_d2[a];
     }
     const int64_t nx = P->n[0], rows = P->n[1] * P->n[2];
-    // the aligned tiles' edge-node copy: same values, rows of an edge adjacent
-    const int64_t ny = P->n[1], nz = P->ndim == 3 ? P->n[2] : 1;
     const int64_t tiles = (nx + awcpml::kTileX - 1) / awcpml::kTileX;
-    std::vector<double> fe((size_t)P->fe_elems);
-    for (int64_t k = 0; k < (P->ndim == 3 ? nz : ny); ++k)
-        for (int64_t t = 0; t < tiles; ++t)
-            for (int s = 0; s < 2; ++s) {
-                int64_t x = s == 0 ? t * awcpml::kTileX - 1 : t * awcpml::kTileX + awcpml::kTileX;
-                x = x < 1 ? 1 : (x > nx - 2 ? nx - 2 : x);
-                if (P->ndim == 3) {
-                    for (int64_t j = 0; j < ny; ++j)
-                        fe[(size_t)(((k * tiles + t) * 2 + s) * ny + j)] = fact[x + nx * (j + ny * k)];
-                } else {
-                    fe[(size_t)((k * tiles + t) * 2 + s)] = fact[x + nx * k];
-                }
-            }
+    const unsigned fe_blocks = (unsigned)std::min<int64_t>((P->fe_elems + 255) / 256, 4096);
     if (P->dtype == AWCPML_F64) {
-        HIP_TRY(hipMemcpy2DAsync(P->fact, P->px * 8, fact, nx * 8, nx * 8, rows, hipMemcpyHostToDevice,
-                                 P->stream));
-        HIP_TRY(hipMemcpyAsync(P->fact_edge, fe.data(), fe.size() * 8, hipMemcpyHostToDevice, P->stream));
+        if ((st = upload_rows_t<double>(P, (double*)P->fact, fact, nx, P->px, rows))) return st;
+        awcpml::gather_fact_edge<double><<<dim3(fe_blocks), dim3(256), 0, P->stream>>>(
+            (const double*)P->fact, (double*)P->fact_edge, nx, P->px, P->n[1], tiles, P->ndim == 3, P->fe_elems);
     } else {
-        std::vector<float> tmp((size_t)nx * rows);
-        for (size_t q = 0; q < tmp.size(); ++q) tmp[q] = (float)fact[q];
-        HIP_TRY(hipMemcpy2DAsync(P->fact, P->px * 4, tmp.data(), nx * 4, nx * 4, rows, hipMemcpyHostToDevice,
-                                 P->stream));
-        std::vector<float> fe32(fe.size());
-        for (size_t q = 0; q < fe.size(); ++q) fe32[q] = (float)fe[q];
-        HIP_TRY(hipMemcpyAsync(P->fact_edge, fe32.data(), fe32.size() * 4, hipMemcpyHostToDevice, P->stream));
+        if ((st = upload_rows_t<float>(P, (float*)P->fact, fact, nx, P->px, rows))) return st;
+        awcpml::gather_fact_edge<float><<<dim3(fe_blocks), dim3(256), 0, P->stream>>>(
+            (const float*)P->fact, (float*)P->fact_edge, nx, P->px, P->n[1], tiles, P->ndim == 3, P->fe_elems);
     }
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(P->stream));
     P->model_set = true;
     ++P->gen;
@@ -1529,19 +1636,8 @@ int awcpml_get_traces(awcpml_plan* P, int shot, double* out) {
     if (!out) return fail(AWCPML_ERR_ARG, "out is NULL");
     int64_t first = 0;
     for (int s = 0; s < shot; ++s) first += (int64_t)P->rec_lin[s].size();
-    const size_t count = (size_t)nrec * P->nt;
-    if (P->dtype == AWCPML_F64) {
-        HIP_TRY(hipMemcpyAsync(out, (char*)P->d_traces + (size_t)first * P->nt * 8, count * 8,
-                               hipMemcpyDeviceToHost, P->stream));
-        HIP_TRY(hipStreamSynchronize(P->stream));
-    } else {
-        std::vector<float> tmp(count);
-        HIP_TRY(hipMemcpyAsync(tmp.data(), (char*)P->d_traces + (size_t)first * P->nt * 4, count * 4,
-                               hipMemcpyDeviceToHost, P->stream));
-        HIP_TRY(hipStreamSynchronize(P->stream));
-        for (size_t q = 0; q < count; ++q) out[q] = tmp[q];
-    }
-    return AWCPML_OK;
+    const int64_t count = nrec * P->nt;
+    return download_rows(P, out, (const char*)P->d_traces + (size_t)(first * P->nt) * P->esize, count, count, 1);
 }
 
 int awcpml_get_field(awcpml_plan* P, int shot, int which, double* out) {
@@ -1552,18 +1648,7 @@ int awcpml_get_field(awcpml_plan* P, int shot, int which, double* out) {
     if (which < 0 || which > 2) return fail(AWCPML_ERR_ARG, "which must be 0, 1 or 2");
     if (!out) return fail(AWCPML_ERR_ARG, "out is NULL");
     const char* src = (const char*)P->p[(P->rot + which) % 3] + (size_t)shot * P->field_elems * P->esize;
-    const int64_t nx = P->n[0], rows = P->n[1] * P->n[2];
-    if (P->dtype == AWCPML_F64) {
-        HIP_TRY(hipMemcpy2DAsync(out, nx * 8, src, P->px * 8, nx * 8, rows, hipMemcpyDeviceToHost, P->stream));
-        HIP_TRY(hipStreamSynchronize(P->stream));
-    } else {
-        std::vector<float> tmp((size_t)nx * rows);
-        HIP_TRY(hipMemcpy2DAsync(tmp.data(), nx * 4, src, P->px * 4, nx * 4, rows, hipMemcpyDeviceToHost,
-                                 P->stream));
-        HIP_TRY(hipStreamSynchronize(P->stream));
-        for (size_t q = 0; q < tmp.size(); ++q) out[q] = tmp[q];
-    }
-    return AWCPML_OK;
+    return download_rows(P, out, src, P->n[0], P->px, P->n[1] * P->n[2]);
 }
 
 int awcpml_run(awcpml_plan* P, double* traces, double* pend) {
@@ -2460,14 +2545,7 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         }
     }
     const int64_t nx = P->n[0], rows = P->n[1] * P->n[2];
-    if (fold) {
-        std::vector<double> host((size_t)P->field_elems);
-        HIP_TRY(hipMemcpyAsync(host.data(), Bf.grad64, host.size() * 8, hipMemcpyDeviceToHost, P->stream));
-        HIP_TRY(hipStreamSynchronize(P->stream));
-        for (int64_t r = 0; r < rows; ++r)
-            for (int64_t i = 0; i < nx; ++i) fbar[r * nx + i] = host[(size_t)(r * P->px + i)];
-        return AWCPML_OK;
-    }
+    if (fold) return download_rows_t<double>(P, fbar, (const double*)Bf.grad64, nx, P->px, rows);
     if (shape.ngroups_cp > 1) {
         const int64_t nb = (P->field_elems + 255) / 256;
         awcpml::sum_shots<T><<<dim3((unsigned)nb), dim3(256), 0, P->stream>>>((T*)Bf.grad, P->field_elems,
@@ -2475,12 +2553,7 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         HIP_TRY(hipGetLastError());
     }
     if ((st = fold_rq((T*)Bf.grad))) return st;
-    std::vector<T> host((size_t)P->field_elems);
-    HIP_TRY(hipMemcpyAsync(host.data(), Bf.grad, host.size() * sizeof(T), hipMemcpyDeviceToHost, P->stream));
-    HIP_TRY(hipStreamSynchronize(P->stream));
-    for (int64_t r = 0; r < rows; ++r)
-        for (int64_t i = 0; i < nx; ++i) fbar[r * nx + i] = (double)host[(size_t)(r * P->px + i)];
-    return AWCPML_OK;
+    return download_rows_t<T>(P, fbar, (const T*)Bf.grad, nx, P->px, rows);
 }
 
 }  // namespace
