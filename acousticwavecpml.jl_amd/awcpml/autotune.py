@@ -41,11 +41,7 @@ def candidates(plan):
 
 
 def two_step_candidates(plan):
-    """(block_rows, march_len, prefetch) of two-step launches worth timing."""
-    if plan.ndim == 2:
-        n_march = plan.n[1] - 2
-        return [(w, min(n_march, ml), pf) for w in (4, 8) for ml in (16, 32, 64, 128)
-                for pf in (1, 2, 3)]
+    """(block_rows, march_len, prefetch) of 3D two-step launches worth timing."""
     n_march = plan.n[2] - 2
     out = []
     for w in ((16, 8) if plan.dtype != 0 else (8, 4)):
@@ -94,6 +90,18 @@ def _load(path):
         return {}
 
 
+def _ms_per_step(plan, steps=34):
+    """Whole time steps (sources and receivers included) of the plan's current
+    launch configuration, after one untimed run."""
+    n = min(plan.nt, steps)
+    plan.reset()
+    plan.advance(n)
+    plan.reset()
+    ms = plan.time_advance(n) / n
+    plan.reset()
+    return ms
+
+
 def autotune(plan, cands=None, launches=8, cache=DEFAULT_CACHE, use_cache=True):
     """Pick the fastest launch shape for ``plan`` and apply it."""
     key = _key(plan)
@@ -125,7 +133,15 @@ def autotune(plan, cands=None, launches=8, cache=DEFAULT_CACHE, use_cache=True):
     # each shape with aligned 64-node tiles and with 62-node tiles
     aligns = (True, False)
     align0 = plan.two_step_align()
-    for w, ml2, pf2 in (two_step_candidates(plan) if cands is None else []):
+    if plan.ndim == 2 and cands is None and plan.nt:
+        # 2D launches of several steps have one shape and handle sources and
+        # receivers themselves: whole steps are compared
+        single = _ms_per_step(plan)
+        plan.set_time_block(2)
+        multi = _ms_per_step(plan)
+        if multi < single:
+            two.append((best["ms_per_step"] * multi / single, 0, 0, 0, None))
+    for w, ml2, pf2 in (two_step_candidates(plan) if cands is None and plan.ndim == 3 else []):
         try:
             for al in aligns:
                 if al is not None:

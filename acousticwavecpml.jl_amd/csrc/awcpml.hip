@@ -29,6 +29,7 @@
 #include "awcpml.h"
 #include "launch.h"
 #include "stencil_kernels.h"
+#include "tile2d_kernels.h"
 #include "transfer_kernels.h"
 
 using awcpml::StencilArgs;
@@ -134,6 +135,9 @@ struct awcpml_plan {
     void* d_traces = nullptr;
     int64_t n_src_total = 0, n_rec_total = 0;
     bool has_io = false;
+    // 2D: the tile kernel's lists (TileArgs), in one buffer
+    void* d_tile_io = nullptr;
+    size_t tile_src_xy = 0, tile_rec_xy = 0, tile_rec_idx = 0, tile_rec_band = 0;  // byte offsets
 
     int64_t it = 0;   // steps done
     int rot = 0;      // p[rot] = pold, p[rot+1] = pcur, p[rot+2] = pnew
@@ -173,6 +177,8 @@ struct awcpml_plan {
     // two time steps per launch (3D): step t+2's field, psi and xi go to
     // spare buffers, which then trade places with the buffers they replace
     int time_block = 1;
+    bool tb_auto = true;             // awcpml_set_time_block was not called: the library decides
+    bool spare_failed = false;       // ... and the spare buffers did not fit
     int tb_rows = 0, tb_march = 0;   // waves per block, chunk length (0: default)
     int tb_prefetch = 0;             // planes of loads in flight (0: default)
     int tb_align = 1;                // 3D: aligned 64-lane tiles where no CPML slab reaches (FP32 default)
@@ -522,6 +528,54 @@ int launch_io(awcpml_plan* P, int64_t it0) {
     return P->dtype == AWCPML_F64 ? launch_io_t<double>(P, it0) : launch_io_t<float>(P, it0);
 }
 
+// Source nodes and interior receivers as the 2D tile kernel reads them: nodes
+// as x | y << 32, each shot's receivers sorted into bands of rows.
+int sync_tile_io(awcpml_plan* P, const std::vector<int64_t>& slin) {
+    auto pack = [&](int64_t lin) { return (lin % P->px) | (lin / P->px) << 32; };
+    const int bands = (int)((P->n[1] + awcpml::kRecBand - 1) / awcpml::kRecBand);
+    std::vector<int64_t> sxy, rxy;
+    std::vector<int> ridx, rband(1, 0);
+    for (int64_t lin : slin) sxy.push_back(pack(lin));
+    int first = 0;
+    for (int s = 0; s < P->nshots; ++s) {
+        const auto& L = P->rec_lin[s];
+        std::vector<std::vector<int>> by(bands);
+        for (size_t r = 0; r < L.size(); ++r) {
+            const int64_t x = L[r] % P->px, y = L[r] / P->px;
+            // a receiver on a Dirichlet node keeps its zeros
+            if (x >= 1 && x <= P->n[0] - 2 && y >= 1 && y <= P->n[1] - 2)
+                by[(size_t)(y / awcpml::kRecBand)].push_back((int)r);
+        }
+        for (const auto& b : by) {
+            for (int r : b) {
+                rxy.push_back(pack(L[r]));
+                ridx.push_back(first + r);
+            }
+            rband.push_back((int)rxy.size());
+        }
+        first += (int)L.size();
+    }
+    const size_t b0 = sxy.size() * 8, b1 = rxy.size() * 8, b2 = ridx.size() * 4, b3 = rband.size() * 4;
+    P->tile_src_xy = 0;
+    P->tile_rec_xy = b0;
+    P->tile_rec_idx = b0 + b1;
+    P->tile_rec_band = b0 + b1 + b2;
+    std::vector<char> all(b0 + b1 + b2 + b3);
+    auto put = [&](size_t at, const void* v, size_t bytes) {
+        if (bytes) memcpy(all.data() + at, v, bytes);
+    };
+    put(P->tile_src_xy, sxy.data(), b0);
+    put(P->tile_rec_xy, rxy.data(), b1);
+    put(P->tile_rec_idx, ridx.data(), b2);
+    put(P->tile_rec_band, rband.data(), b3);
+    dfree(P->d_tile_io);
+    int st = dalloc(&P->d_tile_io, all.size());
+    if (st) return st;
+    HIP_TRY(hipMemcpyAsync(P->d_tile_io, all.data(), all.size(), hipMemcpyHostToDevice, P->stream));
+    HIP_TRY(hipStreamSynchronize(P->stream));
+    return AWCPML_OK;
+}
+
 // Upload the per-shot source/receiver lists as CSR arrays.
 int sync_io(awcpml_plan* P) {
     if (!P->io_dirty) return AWCPML_OK;
@@ -585,6 +639,7 @@ int sync_io(awcpml_plan* P) {
         P->src_on_boundary = P->src_on_boundary || b;
     }
     P->has_io = (P->n_src_total + P->n_rec_total) > 0;
+    if (P->ndim == 2 && (st = sync_tile_io(P, slin))) return st;
     P->io_dirty = false;
     return AWCPML_OK;
 }
@@ -610,17 +665,24 @@ int do_step(awcpml_plan* P, int64_t it0) {
     return AWCPML_OK;
 }
 
-// Two-step launches can run: spare buffers allocated, every field buffer
-// zero on the Dirichlet nodes, at most kMaxSrc2 sources per shot (staged
-// in LDS), 32-bit byte offsets, and a d(pnew)/d(fact) output (if any) for
-// both steps.  two_ok: they also were requested for the plan.
-bool two_applies(const awcpml_plan* P) {
-    return P->p_spare && (!P->q_cur || P->q_next) && !P->src_on_boundary &&
-           P->src_per_shot_max <= awcpml::kMaxSrc2 && !P->boundary_dirty && !P->wide &&
-           (uint64_t)P->field_elems * P->esize < (1ull << 32);
+// Launches of several steps can run: spare buffers allocated, every field
+// buffer zero on the Dirichlet nodes, at most kMaxSrc2 sources per shot, and
+// 32-bit byte offsets.  two_applies: two-step launches, which also write
+// d(pnew)/d(fact) only of both steps; two_ok: ... and were requested.
+bool multi_applies(const awcpml_plan* P) {
+    return P->p_spare && !P->src_on_boundary && P->src_per_shot_max <= awcpml::kMaxSrc2 &&
+           !P->boundary_dirty && !P->wide && (uint64_t)P->field_elems * P->esize < (1ull << 32);
 }
 
+bool two_applies(const awcpml_plan* P) { return multi_applies(P) && (!P->q_cur || P->q_next); }
+
 bool two_ok(const awcpml_plan* P) { return P->time_block == 2 && two_applies(P); }
+
+// A 2D plan takes the tile kernel: by the library's own choice, or where
+// two-step launches were requested.
+bool tile_ok(const awcpml_plan* P) {
+    return P->ndim == 2 && (P->tb_auto || P->time_block == 2) && multi_applies(P);
+}
 
 int two_rows_default(int ndim, int dtype) { return ndim == 2 ? 4 : (dtype == AWCPML_F64 ? 8 : 16); }
 
@@ -742,9 +804,87 @@ int launch_stencil2_t(awcpml_plan* P, int64_t it0) {
     L.block = dim3(awcpml::kTileX, W);
     L.lds = (size_t)8 * (P->halo + 1) * sizeof(T);
     L.stream = P->stream;
-    if (P->ndim == 3) awcpml::launch_plan_stencil2<T, 3>(B, L, W, pf);
-    else awcpml::launch_plan_stencil2<T, 2>(B, L, W, pf);
+    awcpml::launch_plan_stencil2<T>(B, L, W, pf);
     HIP_TRY(hipGetLastError());
+    return AWCPML_OK;
+}
+
+// The tiles along one axis (first node org, own nodes of tile t: [t*own,
+// t*own+own) + org) whose span of `span` nodes, kTileHalo before the owned
+// ones, holds only interior nodes outside the axis's slabs: [*lo, *hi).
+void plain_tiles(const awcpml_plan* P, int a, int64_t org, int64_t own, int64_t span, int tiles, int* lo,
+                 int* hi) {
+    const int64_t first = P->active[a][0] ? P->halo + 1 : 1;
+    const int64_t last = P->active[a][1] ? P->n[a] - P->halo - 2 : P->n[a] - 2;
+    *lo = *hi = 0;
+    for (int t = 0; t < tiles; ++t) {
+        const int64_t c0 = org + t * own - awcpml::kTileHalo, c1 = c0 + span - 1;
+        if (c0 < first || c1 > last) continue;
+        if (*hi == 0) *lo = t;
+        *hi = t + 1;
+    }
+}
+
+// Up to kTileSteps steps of a 2D plan from step it0 in one launch (two where
+// the grid has many tiles without CPML nodes).  q: optional d(pnew)/d(fact)
+// outputs, one field after another.
+template <typename T>
+int launch_tile_t(awcpml_plan* P, int64_t it0, int steps, void* q, bool io = true) {
+    awcpml::TileArgs<T> B;
+    memset(&B, 0, sizeof B);
+    B.s = make_args<T>(P, P->rot, P->par);
+    for (int a = 0; a < 2; ++a)
+        for (int s = 0; s < 2; ++s) {
+            B.s.side[a][s].psi_wr = (T*)P->psi_spare[a][s];
+            B.xi_out[a][s] = (T*)P->xi_spare[a][s];
+        }
+    B.p1 = (T*)P->p[(P->rot + 2) % 3];
+    B.p2 = (T*)P->p_spare;
+    B.q = (T*)q;
+    B.q_step = P->field_elems * P->nshots;
+    const char* lists = (const char*)P->d_tile_io;
+    B.src_xy = (const int64_t*)(lists + P->tile_src_xy);
+    B.src_wav = (const T*)P->d_src_wav;
+    B.src_start = (const int*)P->d_src_start;
+    B.rec_xy = (const int64_t*)(lists + P->tile_rec_xy);
+    B.rec_idx = (const int*)(lists + P->tile_rec_idx);
+    B.rec_band = (const int*)(lists + P->tile_rec_band);
+    B.bands = (int)((P->n[1] + awcpml::kRecBand - 1) / awcpml::kRecBand);
+    B.traces = (T*)P->d_traces;
+    B.nt = P->nt;
+    B.it0 = it0;
+    B.steps = steps;
+    B.io = io;
+    constexpr int64_t H = awcpml::kTileHalo, OX = awcpml::kTileOwnX;
+    B.tiles_x = (int)((P->n[0] - 2) / OX + 1);
+    auto shape = [&](int rows) { B.tiles_y = (int)((P->n[1] - 2 + rows - 2 * H - 1) / (rows - 2 * H)); };
+    int rows = 64;
+    shape(rows);
+    bool overlap = false;  // some axis's slabs overlap
+    for (int a = 0; a < 2; ++a)
+        overlap = overlap || ((P->active[a][0] || P->active[a][1]) && P->n[a] < 2 * (int64_t)P->halo + 3);
+    if (overlap || (int64_t)B.tiles_x * B.tiles_y * P->nshots < 512) shape(rows = 32);
+    bool split = false;
+    if (rows == 64) {
+        plain_tiles(P, 0, 0, OX, awcpml::kTileX, B.tiles_x, &B.ix0, &B.ix1);
+        plain_tiles(P, 1, 1, rows - 2 * H, rows, B.tiles_y, &B.iy0, &B.iy1);
+        split = (int64_t)(B.ix1 - B.ix0) * (B.iy1 - B.iy0) * P->nshots >= 1024;
+        if (!split) B.ix0 = B.ix1 = B.iy0 = B.iy1 = 0;
+    }
+    const int64_t plain = (int64_t)(B.ix1 - B.ix0) * (B.iy1 - B.iy0);
+    for (int part = split ? 0 : 1; part < 2; ++part) {
+        const int64_t n = (part ? (int64_t)B.tiles_x * B.tiles_y - plain : plain) * P->nshots;
+        if (n == 0) continue;
+        B.logical_blocks = (int)n;
+        B.grid_blocks = (int)round_up(n, awcpml::kNumXcd);
+        awcpml::LaunchShape L;
+        L.grid = dim3(B.grid_blocks);
+        L.lds = 0;
+        L.stream = P->stream;
+        awcpml::launch_plan_tile2d<T>(
+            B, L, rows, part == 0 ? awcpml::kTilePlain : overlap ? awcpml::kTileOverlap : awcpml::kTileSlabs);
+        HIP_TRY(hipGetLastError());
+    }
     return AWCPML_OK;
 }
 
@@ -789,22 +929,49 @@ int do_step2(awcpml_plan* P, int64_t it0) {
     return AWCPML_OK;
 }
 
-// Enqueue the steps it0 .. it0+n-1 (pairs in two-step launches where they
-// apply), advancing the host's layout state as they are enqueued.
-int enqueue_steps(awcpml_plan* P, int64_t it0, int64_t n) {
-    const bool two = two_ok(P);
-    for (int64_t q = 0; q < n;) {
-        int st;
-        if (two && n - q >= 2) {
-            st = do_step2(P, it0 + q);
-            q += 2;
+int do_tile(awcpml_plan* P, int64_t it0, int steps, void* q) {
+    const int st = P->dtype == AWCPML_F64 ? launch_tile_t<double>(P, it0, steps, q)
+                                          : launch_tile_t<float>(P, it0, steps, q);
+    if (!st) two_swap(P);
+    return st;
+}
+
+// Steps of the next launch of a 2D plan with `left` steps to go: near-equal
+// launches of at most kTileSteps.  keep: the run ends with a two-step launch,
+// after which all three field buffers hold what single steps leave in them
+// (a longer one leaves the pressure of its first step in place of the
+// reference's stale pnew).
+int tile_steps(int64_t left, bool keep) {
+    if (left <= 2) return (int)left;
+    const int64_t rest = keep ? left - 2 : left;
+    const int64_t launches = (rest + awcpml::kTileSteps - 1) / awcpml::kTileSteps;
+    return (int)((rest + launches - 1) / launches);
+}
+
+// Enqueue the steps it0 .. it0+n-1 (several per launch where that applies),
+// advancing the host's layout state as they are enqueued.  q: d(pnew)/d(fact)
+// outputs of the steps, one field of all shots after another, or null.
+int enqueue_steps(awcpml_plan* P, int64_t it0, int64_t n, bool keep = true, char* q = nullptr) {
+    const bool tile = tile_ok(P);
+    const size_t fb = (size_t)P->field_elems * P->nshots * P->esize;
+    int st = AWCPML_OK;
+    for (int64_t s = 0; s < n && !st;) {
+        const int64_t left = n - s;
+        char* const qs = q ? q + (size_t)s * fb : nullptr;
+        int take = tile ? tile_steps(left, keep) : 1;
+        if (take >= 2) {
+            st = do_tile(P, it0 + s, take, qs);
         } else {
-            st = do_step(P, it0 + q);
-            q += 1;
+            P->q_cur = qs;
+            P->q_next = qs && left >= 2 ? qs + fb : nullptr;
+            if (!tile && left >= 2 && two_ok(P)) take = 2;
+            else P->q_next = nullptr;
+            st = take == 2 ? do_step2(P, it0 + s) : do_step(P, it0 + s);
+            P->q_cur = P->q_next = nullptr;
         }
-        if (st) return st;
+        s += take;
     }
-    return AWCPML_OK;
+    return st;
 }
 
 // Capture `n` steps starting at step it0 on `stream` into an executable
@@ -870,11 +1037,72 @@ int plan_graph(awcpml_plan* P, int64_t n, GraphEntry** out) {
     return AWCPML_OK;
 }
 
+// The spare buffers of multi-step launches (one field, one psi and one xi per
+// CPML side).  They start as zeros, like every buffer after a reset, and are
+// allocated before any such launch, so the layout is still home.
+int alloc_spares(awcpml_plan* P) {
+    if (P->p_spare) return AWCPML_OK;
+    const size_t fbytes = (size_t)P->field_elems * P->nshots * P->esize;
+    void* f = nullptr;
+    void* psi[3][2] = {};
+    void* xi[3][2] = {};
+    int st = dalloc(&f, fbytes);
+    for (int a = 0; a < P->ndim && !st; ++a)
+        for (int s = 0; s < 2 && !st; ++s) {
+            st = dalloc(&psi[a][s], (size_t)P->psi_elems[a] * P->nshots * P->esize);
+            if (!st) st = dalloc(&xi[a][s], (size_t)P->xi_elems[a] * P->nshots * P->esize);
+        }
+    auto clear = [&](void* v, size_t bytes) {
+        if (!st && bytes && hipMemsetAsync(v, 0, bytes, P->stream) != hipSuccess)
+            st = fail(AWCPML_ERR_HIP, "hipMemsetAsync failed");
+    };
+    clear(f, fbytes);
+    for (int a = 0; a < P->ndim; ++a)
+        for (int s = 0; s < 2; ++s) {
+            clear(psi[a][s], (size_t)P->psi_elems[a] * P->nshots * P->esize);
+            clear(xi[a][s], (size_t)P->xi_elems[a] * P->nshots * P->esize);
+        }
+    if (!st && hipStreamSynchronize(P->stream) != hipSuccess)
+        st = fail(AWCPML_ERR_HIP, "hipStreamSynchronize failed");
+    if (st) {
+        dfree(f);
+        for (int a = 0; a < 3; ++a)
+            for (int s = 0; s < 2; ++s) {
+                dfree(psi[a][s]);
+                dfree(xi[a][s]);
+            }
+        return st;
+    }
+    P->p_spare = f;
+    P->home.p[3] = f;
+    for (int a = 0; a < 3; ++a)
+        for (int s = 0; s < 2; ++s) {
+            P->home.psi[a][s][2] = P->psi_spare[a][s] = psi[a][s];
+            P->home.xi[a][s][1] = P->xi_spare[a][s] = xi[a][s];
+        }
+    ++P->gen;
+    return AWCPML_OK;
+}
+
+// A plan left to the library's choice gets its spare buffers with its first
+// run of several steps; where they do not fit it keeps single steps.
+int auto_spares(awcpml_plan* P, int64_t n) {
+    if (!P->tb_auto || P->ndim != 2 || n < 2 || P->p_spare || P->spare_failed) return AWCPML_OK;
+    const int st = alloc_spares(P);
+    if (st != AWCPML_ERR_NOMEM) return st;
+    (void)hipGetLastError();
+    g_err.clear();
+    P->spare_failed = true;
+    return AWCPML_OK;
+}
+
 // Enqueue n steps from the plan's current state (no synchronisation).  With
 // graphs enabled the sequence is captured once per (first step, length,
 // buffer layout) and replayed afterwards.
 int run_steps(awcpml_plan* P, int64_t n) {
     if (n <= 0) return AWCPML_OK;
+    int sp = auto_spares(P, n);
+    if (sp) return sp;
     if (P->use_graph) {
         GraphEntry* g = nullptr;
         int st = plan_graph(P, n, &g);
@@ -1460,6 +1688,7 @@ int awcpml_plan_destroy(awcpml_plan* P) {
     dfree(P->d_rec_lin);
     dfree(P->d_rec_start);
     dfree(P->d_traces);
+    dfree(P->d_tile_io);
     dfree(P->ck);
     if (P->stage) (void)hipFree(P->stage);
     if (P->stream) (void)hipStreamDestroy(P->stream);
@@ -1772,29 +2001,8 @@ int awcpml_set_time_block(awcpml_plan* P, int steps, int block_rows, int march_l
         return fail(AWCPML_ERR_ARG, "block_rows must be 0, 4 or 8 for 2D plans (got %d)", block_rows);
     if (march_len < 0) return fail(AWCPML_ERR_ARG, "march_len < 0");
     if (prefetch < 0 || prefetch > 3) return fail(AWCPML_ERR_ARG, "prefetch must be 0..3 (got %d)", prefetch);
-    if (steps == 2 && !P->p_spare) {
-        // spares start as zeros, like every buffer after a reset; a spare is
-        // allocated before any two-step launch, so the layout is still home
-        const size_t fbytes = (size_t)P->field_elems * P->nshots * P->esize;
-        if ((st = dalloc(&P->p_spare, fbytes))) return st;
-        HIP_TRY(hipMemsetAsync(P->p_spare, 0, fbytes, P->stream));
-        for (int a = 0; a < P->ndim; ++a)
-            for (int s = 0; s < 2; ++s) {
-                const size_t pb = (size_t)P->psi_elems[a] * P->nshots * P->esize;
-                const size_t xb = (size_t)P->xi_elems[a] * P->nshots * P->esize;
-                if ((st = dalloc(&P->psi_spare[a][s], pb))) return st;
-                if ((st = dalloc(&P->xi_spare[a][s], xb))) return st;
-                HIP_TRY(hipMemsetAsync(P->psi_spare[a][s], 0, pb, P->stream));
-                if (xb) HIP_TRY(hipMemsetAsync(P->xi_spare[a][s], 0, xb, P->stream));
-            }
-        HIP_TRY(hipStreamSynchronize(P->stream));
-        P->home.p[3] = P->p_spare;
-        for (int a = 0; a < 3; ++a)
-            for (int s = 0; s < 2; ++s) {
-                P->home.psi[a][s][2] = P->psi_spare[a][s];
-                P->home.xi[a][s][1] = P->xi_spare[a][s];
-            }
-    }
+    if (steps == 2 && (st = alloc_spares(P))) return st;
+    P->tb_auto = false;
     P->time_block = steps;
     P->tb_rows = block_rows;
     P->tb_march = march_len;
@@ -1811,7 +2019,7 @@ int awcpml_get_time_block(const awcpml_plan* P, int* steps, int* block_rows, int
     int W, ml, pf;
     two_tiling(P, &W, &ml, &pf);
     // the steps a launch advances now (1 where two-step launches do not apply)
-    *steps = two_ok(P) ? 2 : 1;
+    *steps = two_ok(P) || tile_ok(P) ? 2 : 1;
     *block_rows = W;
     *march_len = ml;
     *prefetch = pf;
@@ -1846,7 +2054,11 @@ int awcpml_time_stencil2(awcpml_plan* P, int nlaunches, double* ms_total) {
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, P->stream));
     for (int q = 0; q < nlaunches; ++q) {
-        st = P->dtype == AWCPML_F64 ? launch_stencil2_t<double>(P, 0) : launch_stencil2_t<float>(P, 0);
+        const bool f64 = P->dtype == AWCPML_F64;
+        if (P->ndim == 2)
+            st = f64 ? launch_tile_t<double>(P, 0, 2, nullptr, false) : launch_tile_t<float>(P, 0, 2, nullptr, false);
+        else
+            st = f64 ? launch_stencil2_t<double>(P, 0) : launch_stencil2_t<float>(P, 0);
         if (st) break;
         two_swap(P);
     }
@@ -1874,7 +2086,9 @@ int awcpml_batch_create(awcpml_plan* const* plans, int count, awcpml_batch** out
             return fail(AWCPML_ERR_ARG, "plans of a batch must share ndim and dtype (plan %d differs)", q);
         int st = ready(plans[q]);
         if (st) return st;
-        if (!at_home(plans[q]))
+        // (a plan left to the library's choice of launches runs nothing in the
+        // batch before awcpml_batch_reset brings it home)
+        if (!at_home(plans[q]) && !plans[q]->tb_auto)
             return fail(AWCPML_ERR_STATE,
                         "plan %d's buffers traded roles in two-step launches (alone or in a batch) "
                         "since its last reset: reset it before batching", q);
@@ -2500,17 +2714,9 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     for (int64_t seg = P->ck_count - 1; seg >= 0; --seg) {
         const int64_t c0 = seg * K, c1 = std::min<int64_t>(c0 + K, nt);
         if ((st = ck_copy(P, seg, false))) return st;
-        for (int64_t s = c0 + 1; s <= c1;) {  // replay, storing q^s
-            P->q_cur = (char*)Bf.q + (size_t)(s - c0 - 1) * fb;
-            P->q_next = s + 1 <= c1 ? (char*)Bf.q + (size_t)(s - c0) * fb : nullptr;
-            const int64_t n = P->q_next && two_ok(P) ? 2 : 1;  // bit-identical q either way
-            if (n == 1) P->q_next = nullptr;
-            st = n == 2 ? do_step2(P, s - 1) : do_step(P, s - 1);
-            P->q_cur = P->q_next = nullptr;
-            if (st) return st;
-            P->it += n;
-            s += n;
-        }
+        // replay, storing q^s (bit-identical whatever the steps per launch)
+        if ((st = enqueue_steps(P, c0, c1 - c0, false, (char*)Bf.q))) return st;
+        P->it = c1;
         for (int64_t s = c1; s > c0; --s) {
             const void* q = (const char*)Bf.q + (size_t)(s - c0 - 1) * fb;
             awcpml::AdjointArgs<T> A;
@@ -2588,8 +2794,8 @@ int awcpml_checkpoint_run(awcpml_plan* P, int64_t every) {
     for (int64_t c = 0; c < count; ++c) {
         if ((st = ck_copy(P, c, true))) return st;
         const int64_t n = std::min<int64_t>(every, P->nt - P->it);
-        // two steps per launch where the plan takes them (bit-identical)
-        if ((st = enqueue_steps(P, P->it, n))) return st;
+        // several steps per launch where the plan takes them (bit-identical)
+        if ((st = enqueue_steps(P, P->it, n, c == count - 1))) return st;
         P->it += n;
     }
     HIP_TRY(hipStreamSynchronize(P->stream));

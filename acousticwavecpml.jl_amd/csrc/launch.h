@@ -11,6 +11,9 @@
 
 namespace awcpml {
 
+template <typename T>
+struct TileArgs;  // tile2d_kernels.h
+
 struct LaunchShape {
     dim3 grid, block;
     size_t lds;          // dynamic LDS bytes (march-axis CPML coefficients)
@@ -25,12 +28,18 @@ void launch_plan_stencil(const StencilArgs<T>& A, const LaunchShape& L, int pipe
 template <typename T, int NDIM>
 void launch_batch_stencil(const BatchArgs<T>& A, const LaunchShape& L, int pipe, bool off64);
 
-// Two time steps per launch; rows: waves per block (3D: 4, 8, 16 rows of a
-// tile; 2D: 4 or 8 march chunks); pf: march positions of loads in flight
-// per wave (1..3).
-template <typename T, int NDIM>
+// Two time steps per launch of a 3D plan; rows: waves per block (4, 8, 16
+// rows of a tile); pf: planes of loads in flight per wave (1..3).
+template <typename T>
 void launch_plan_stencil2(const Stencil2Args<T>& B, const LaunchShape& L, int rows, int pf);
 
+// Up to kTileSteps time steps of a 2D plan per launch.  rows: the tile's rows
+// (32 or 64; kTileOverlap: 32); kind: a TileKind.
+template <typename T>
+void launch_plan_tile2d(const TileArgs<T>& B, const LaunchShape& L, int rows, int kind);
+
+// The same for a batch (2D: rows is the number of march chunks per block, 4
+// or 8).
 template <typename T, int NDIM>
 void launch_batch_stencil2(const Batch2Args<T>& B, const LaunchShape& L, int rows, int pf);
 

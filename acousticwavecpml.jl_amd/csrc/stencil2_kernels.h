@@ -1359,13 +1359,6 @@ __global__ __launch_bounds__(64 * W) void stencil3d_two(const Stencil2Args<T> B)
     stencil3d_two_block<T, Off, W, PF>(B, B.it0, lb);
 }
 
-template <typename T, typename Off, int BY, int PF>
-__global__ __launch_bounds__(64 * BY) void stencil2d_two(const Stencil2Args<T> B) {
-    const int lb = logical_block(blockIdx.x, B.s.grid_blocks);
-    if (lb >= B.s.logical_blocks) return;  // whole block
-    stencil2d_two_block<T, Off, BY, PF>(B, B.it0, lb);
-}
-
 template <typename T, typename Off, int W, int PF>
 __global__ __launch_bounds__(64 * W) void stencil3d_two_batch(const Batch2Args<T> B) {
     const int lb = logical_block(blockIdx.x, B.grid_blocks);
