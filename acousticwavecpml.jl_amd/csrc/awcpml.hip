@@ -97,6 +97,20 @@ void drop_graphs(std::vector<GraphEntry>& g) {
 
 }  // namespace
 
+// Several device buffers in one allocation (or, above kGroupBytes, each in its
+// own: there the allocations' time no longer matters and smaller pieces fit
+// better).  A plan of some forty separate buffers spent up to 3.6 ms on
+// hipMalloc and hipFree, which wait for the device, and cleared them with 20-30
+// fills: 101x91x83 FP64, one plan and 160 steps, 9.7 ms apart and 7.3 ms
+// together.
+struct BufferGroup {
+    void* base = nullptr;
+    size_t bytes = 0;
+    bool holds(const void* p) const {
+        return base && (const char*)p >= (const char*)base && (const char*)p < (const char*)base + bytes;
+    }
+};
+
 struct awcpml_plan {
     int ndim = 0, dtype = 0, nshots = 0, halo = 0;
     int64_t n[3] = {1, 1, 1};
@@ -135,13 +149,19 @@ struct awcpml_plan {
     void* d_traces = nullptr;
     int64_t n_src_total = 0, n_rec_total = 0;
     bool has_io = false;
-    // 2D: the tile kernel's lists (TileArgs), in one buffer
-    void* d_tile_io = nullptr;
-    size_t tile_src_xy = 0, tile_rec_xy = 0, tile_rec_idx = 0, tile_rec_band = 0;  // byte offsets
+    // source and receiver lists in one buffer; 2D: the tile kernel's
+    // (TileArgs) among them, at these byte offsets
+    void* d_io_lists = nullptr;
+    size_t tile_src_xy = 0, tile_rec_xy = 0, tile_rec_idx = 0, tile_rec_band = 0;
 
     int64_t it = 0;   // steps done
     int rot = 0;      // p[rot] = pold, p[rot+1] = pcur, p[rot+2] = pnew
     int par = 0;      // psi[..][par] = previous step
+
+    // the buffers above: fields, psi and xi first (state_bytes), then the
+    // model and coefficients; the spares; sources, receivers and traces
+    BufferGroup main, spares, io;
+    size_t state_bytes = 0;
 
     // dense FP64 rows on their way to or from the host (transfer_kernels.h),
     // allocated on first use
@@ -257,6 +277,54 @@ int dalloc(void** ptr, size_t bytes) {
 void dfree(void*& ptr) {
     if (ptr) (void)hipFree(ptr);
     ptr = nullptr;
+}
+
+constexpr size_t kGroupBytes = 2ull << 30;
+constexpr size_t kGroupAlign = 4096;
+
+// A list of buffers to allocate together: each pointer and its size.
+struct GroupList {
+    std::vector<std::pair<void**, size_t>> want;
+    size_t total = 0;
+    void add(void** p, size_t bytes) {
+        want.push_back({p, bytes});
+        total += (std::max<size_t>(bytes, 256) + kGroupAlign - 1) / kGroupAlign * kGroupAlign;
+    }
+};
+
+void group_free(BufferGroup& G, GroupList& L) {
+    for (auto& w : L.want) {
+        if (!G.holds(*w.first)) dfree(*w.first);
+        *w.first = nullptr;
+    }
+    dfree(G.base);
+    G.bytes = 0;
+}
+
+// Allocate every buffer of L, in order, in one block where that is small
+// enough; on failure none is left.
+int group_alloc(BufferGroup& G, GroupList& L) {
+    if (L.total <= kGroupBytes) {
+        const int st = dalloc(&G.base, L.total);
+        if (st) return st;
+        G.bytes = L.total;
+        char* at = (char*)G.base;
+        for (auto& w : L.want) {
+            *w.first = at;
+            at += (std::max<size_t>(w.second, 256) + kGroupAlign - 1) / kGroupAlign * kGroupAlign;
+        }
+        return AWCPML_OK;
+    }
+    for (auto& w : L.want) {
+        const int st = dalloc(w.first, w.second);
+        if (st) {
+            const std::string keep = g_err;
+            for (auto& v : L.want) dfree(*v.first);
+            g_err = keep;
+            return st;
+        }
+    }
+    return AWCPML_OK;
 }
 
 // Staged transfers take at most this many FP64 values at a time (32 MiB per
@@ -528,9 +596,19 @@ int launch_io(awcpml_plan* P, int64_t it0) {
     return P->dtype == AWCPML_F64 ? launch_io_t<double>(P, it0) : launch_io_t<float>(P, it0);
 }
 
+void io_free(awcpml_plan* P) {
+    GroupList L;
+    L.add(&P->d_io_lists, 0);
+    L.add(&P->d_src_wav, 0);
+    L.add(&P->d_traces, 0);
+    group_free(P->io, L);
+    P->d_src_lin = P->d_src_start = P->d_src_seq = P->d_rec_lin = P->d_rec_start = nullptr;
+}
+
 // Source nodes and interior receivers as the 2D tile kernel reads them: nodes
 // as x | y << 32, each shot's receivers sorted into bands of rows.
-int sync_tile_io(awcpml_plan* P, const std::vector<int64_t>& slin) {
+template <typename Put>
+void tile_lists(awcpml_plan* P, const std::vector<int64_t>& slin, Put put) {
     auto pack = [&](int64_t lin) { return (lin % P->px) | (lin / P->px) << 32; };
     const int bands = (int)((P->n[1] + awcpml::kRecBand - 1) / awcpml::kRecBand);
     std::vector<int64_t> sxy, rxy;
@@ -539,41 +617,28 @@ int sync_tile_io(awcpml_plan* P, const std::vector<int64_t>& slin) {
     int first = 0;
     for (int s = 0; s < P->nshots; ++s) {
         const auto& L = P->rec_lin[s];
-        std::vector<std::vector<int>> by(bands);
+        std::vector<std::pair<int64_t, int>> in;  // (band, receiver)
         for (size_t r = 0; r < L.size(); ++r) {
             const int64_t x = L[r] % P->px, y = L[r] / P->px;
             // a receiver on a Dirichlet node keeps its zeros
             if (x >= 1 && x <= P->n[0] - 2 && y >= 1 && y <= P->n[1] - 2)
-                by[(size_t)(y / awcpml::kRecBand)].push_back((int)r);
+                in.push_back({y / awcpml::kRecBand, (int)r});
         }
-        for (const auto& b : by) {
-            for (int r : b) {
-                rxy.push_back(pack(L[r]));
-                ridx.push_back(first + r);
+        std::sort(in.begin(), in.end());
+        size_t e = 0;
+        for (int b = 0; b < bands; ++b) {
+            for (; e < in.size() && in[e].first == b; ++e) {
+                rxy.push_back(pack(L[(size_t)in[e].second]));
+                ridx.push_back(first + in[e].second);
             }
             rband.push_back((int)rxy.size());
         }
         first += (int)L.size();
     }
-    const size_t b0 = sxy.size() * 8, b1 = rxy.size() * 8, b2 = ridx.size() * 4, b3 = rband.size() * 4;
-    P->tile_src_xy = 0;
-    P->tile_rec_xy = b0;
-    P->tile_rec_idx = b0 + b1;
-    P->tile_rec_band = b0 + b1 + b2;
-    std::vector<char> all(b0 + b1 + b2 + b3);
-    auto put = [&](size_t at, const void* v, size_t bytes) {
-        if (bytes) memcpy(all.data() + at, v, bytes);
-    };
-    put(P->tile_src_xy, sxy.data(), b0);
-    put(P->tile_rec_xy, rxy.data(), b1);
-    put(P->tile_rec_idx, ridx.data(), b2);
-    put(P->tile_rec_band, rband.data(), b3);
-    dfree(P->d_tile_io);
-    int st = dalloc(&P->d_tile_io, all.size());
-    if (st) return st;
-    HIP_TRY(hipMemcpyAsync(P->d_tile_io, all.data(), all.size(), hipMemcpyHostToDevice, P->stream));
-    HIP_TRY(hipStreamSynchronize(P->stream));
-    return AWCPML_OK;
+    P->tile_src_xy = put(sxy.data(), sxy.size() * 8);
+    P->tile_rec_xy = put(rxy.data(), rxy.size() * 8);
+    P->tile_rec_idx = put(ridx.data(), ridx.size() * 4);
+    P->tile_rec_band = put(rband.data(), rband.size() * 4);
 }
 
 // Upload the per-shot source/receiver lists as CSR arrays.
@@ -599,32 +664,35 @@ int sync_io(awcpml_plan* P) {
     }
     drop_graphs(P->graphs);  // they reference the buffers below
     ++P->gen;                // and so do the argument tables of batches
-    dfree(P->d_src_lin);
-    dfree(P->d_src_wav);
-    dfree(P->d_src_start);
-    dfree(P->d_src_seq);
-    dfree(P->d_rec_lin);
-    dfree(P->d_rec_start);
-    dfree(P->d_traces);
-    int st;
-    if ((st = dalloc(&P->d_src_lin, slin.size() * 8))) return st;
-    if ((st = dalloc(&P->d_src_wav, wav.size() * P->esize))) return st;
-    if ((st = dalloc(&P->d_src_start, sstart.size() * 4))) return st;
-    if ((st = dalloc(&P->d_src_seq, seq.size() * 4))) return st;
-    if ((st = dalloc(&P->d_rec_lin, rlin.size() * 8))) return st;
-    if ((st = dalloc(&P->d_rec_start, rstart.size() * 4))) return st;
-    if ((st = dalloc(&P->d_traces, (size_t)rlin.size() * (size_t)std::max<int64_t>(P->nt, 1) * P->esize)))
-        return st;
-    if (!slin.empty())
-        HIP_TRY(hipMemcpyAsync(P->d_src_lin, slin.data(), slin.size() * 8, hipMemcpyHostToDevice, P->stream));
+    // the lists that are copied as they are, packed for one copy
+    std::vector<char> lists;
+    auto put = [&](const void* v, size_t bytes) {
+        const size_t at = lists.size();
+        lists.resize(at + (bytes + 7) / 8 * 8);
+        if (bytes) memcpy(lists.data() + at, v, bytes);
+        return at;
+    };
+    const size_t at_slin = put(slin.data(), slin.size() * 8), at_rlin = put(rlin.data(), rlin.size() * 8);
+    const size_t at_sstart = put(sstart.data(), sstart.size() * 4), at_rstart = put(rstart.data(), rstart.size() * 4);
+    const size_t at_seq = put(seq.data(), seq.size() * 4);
+    if (P->ndim == 2) tile_lists(P, slin, put);
+    io_free(P);
+    const size_t trace_bytes = (size_t)rlin.size() * (size_t)std::max<int64_t>(P->nt, 0) * P->esize;
+    GroupList L;
+    L.add(&P->d_io_lists, lists.size());
+    L.add(&P->d_src_wav, wav.size() * P->esize);
+    L.add(&P->d_traces, trace_bytes);
+    int st = group_alloc(P->io, L);
+    if (st) return st;
+    char* base = (char*)P->d_io_lists;
+    P->d_src_lin = base + at_slin;
+    P->d_rec_lin = base + at_rlin;
+    P->d_src_start = base + at_sstart;
+    P->d_rec_start = base + at_rstart;
+    P->d_src_seq = base + at_seq;
+    HIP_TRY(hipMemcpyAsync(base, lists.data(), lists.size(), hipMemcpyHostToDevice, P->stream));
     if ((st = upload(P, P->d_src_wav, wav.data(), wav.size()))) return st;
-    HIP_TRY(hipMemcpyAsync(P->d_src_start, sstart.data(), sstart.size() * 4, hipMemcpyHostToDevice, P->stream));
-    HIP_TRY(hipMemcpyAsync(P->d_src_seq, seq.data(), seq.size() * 4, hipMemcpyHostToDevice, P->stream));
-    if (!rlin.empty())
-        HIP_TRY(hipMemcpyAsync(P->d_rec_lin, rlin.data(), rlin.size() * 8, hipMemcpyHostToDevice, P->stream));
-    HIP_TRY(hipMemcpyAsync(P->d_rec_start, rstart.data(), rstart.size() * 4, hipMemcpyHostToDevice, P->stream));
-    if (!rlin.empty() && P->nt > 0)
-        HIP_TRY(hipMemsetAsync(P->d_traces, 0, (size_t)rlin.size() * P->nt * P->esize, P->stream));
+    if (trace_bytes) HIP_TRY(hipMemsetAsync(P->d_traces, 0, trace_bytes, P->stream));
     HIP_TRY(hipStreamSynchronize(P->stream));
     P->n_src_total = (int64_t)slin.size();
     P->n_rec_total = (int64_t)rlin.size();
@@ -639,7 +707,6 @@ int sync_io(awcpml_plan* P) {
         P->src_on_boundary = P->src_on_boundary || b;
     }
     P->has_io = (P->n_src_total + P->n_rec_total) > 0;
-    if (P->ndim == 2 && (st = sync_tile_io(P, slin))) return st;
     P->io_dirty = false;
     return AWCPML_OK;
 }
@@ -842,7 +909,7 @@ int launch_tile_t(awcpml_plan* P, int64_t it0, int steps, void* q, bool io = tru
     B.p2 = (T*)P->p_spare;
     B.q = (T*)q;
     B.q_step = P->field_elems * P->nshots;
-    const char* lists = (const char*)P->d_tile_io;
+    const char* lists = (const char*)P->d_io_lists;
     B.src_xy = (const int64_t*)(lists + P->tile_src_xy);
     B.src_wav = (const T*)P->d_src_wav;
     B.src_start = (const int*)P->d_src_start;
@@ -1042,36 +1109,29 @@ int plan_graph(awcpml_plan* P, int64_t n, GraphEntry** out) {
 // allocated before any such launch, so the layout is still home.
 int alloc_spares(awcpml_plan* P) {
     if (P->p_spare) return AWCPML_OK;
-    const size_t fbytes = (size_t)P->field_elems * P->nshots * P->esize;
     void* f = nullptr;
     void* psi[3][2] = {};
     void* xi[3][2] = {};
-    int st = dalloc(&f, fbytes);
-    for (int a = 0; a < P->ndim && !st; ++a)
-        for (int s = 0; s < 2 && !st; ++s) {
-            st = dalloc(&psi[a][s], (size_t)P->psi_elems[a] * P->nshots * P->esize);
-            if (!st) st = dalloc(&xi[a][s], (size_t)P->xi_elems[a] * P->nshots * P->esize);
-        }
-    auto clear = [&](void* v, size_t bytes) {
-        if (!st && bytes && hipMemsetAsync(v, 0, bytes, P->stream) != hipSuccess)
-            st = fail(AWCPML_ERR_HIP, "hipMemsetAsync failed");
-    };
-    clear(f, fbytes);
+    GroupList L;
+    L.add(&f, (size_t)P->field_elems * P->nshots * P->esize);
     for (int a = 0; a < P->ndim; ++a)
         for (int s = 0; s < 2; ++s) {
-            clear(psi[a][s], (size_t)P->psi_elems[a] * P->nshots * P->esize);
-            clear(xi[a][s], (size_t)P->xi_elems[a] * P->nshots * P->esize);
+            L.add(&psi[a][s], (size_t)P->psi_elems[a] * P->nshots * P->esize);
+            L.add(&xi[a][s], (size_t)P->xi_elems[a] * P->nshots * P->esize);
         }
-    if (!st && hipStreamSynchronize(P->stream) != hipSuccess)
-        st = fail(AWCPML_ERR_HIP, "hipStreamSynchronize failed");
-    if (st) {
-        dfree(f);
-        for (int a = 0; a < 3; ++a)
-            for (int s = 0; s < 2; ++s) {
-                dfree(psi[a][s]);
-                dfree(xi[a][s]);
-            }
-        return st;
+    int st = group_alloc(P->spares, L);
+    if (st) return st;
+    hipError_t e = hipSuccess;
+    if (P->spares.base) {
+        e = hipMemsetAsync(P->spares.base, 0, P->spares.bytes, P->stream);
+    } else {
+        for (auto& w : L.want)
+            if (e == hipSuccess && w.second) e = hipMemsetAsync(*w.first, 0, w.second, P->stream);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(P->stream);
+    if (e != hipSuccess) {
+        group_free(P->spares, L);
+        return fail(AWCPML_ERR_HIP, "clearing the spare buffers failed: %s", hipGetErrorString(e));
     }
     P->p_spare = f;
     P->home.p[3] = f;
@@ -1627,23 +1687,26 @@ int awcpml_plan_create(int ndim, int64_t nx, int64_t ny, int64_t nz, int halo, i
         return fail(AWCPML_ERR_HIP, "hipStreamCreate failed: %s", hipGetErrorString(he));
     }
     const size_t fbytes = (size_t)P->field_elems * nshots * P->esize;
-    for (int b = 0; b < 3 && !st; ++b) st = dalloc(&P->p[b], fbytes);
-    if (!st) st = dalloc(&P->fact, (size_t)P->field_elems * P->esize);
-    {
-        const int64_t tiles = (nx + awcpml::kTileX - 1) / awcpml::kTileX;
-        P->fe_elems = ndim == 3 ? nz * tiles * 2 * ny : ny * tiles * 2;
-        if (!st) st = dalloc(&P->fact_edge, (size_t)P->fe_elems * P->esize);
-    }
-    for (int a = 0; a < ndim && !st; ++a) {
+    GroupList L;
+    for (int b = 0; b < 3; ++b) L.add(&P->p[b], fbytes);
+    for (int a = 0; a < ndim; ++a) {
         P->psi_elems[a] = slab_elems(P, a, halo + 1);
         P->xi_elems[a] = slab_elems(P, a, halo);
-        for (int s = 0; s < 2 && !st; ++s) {
-            st = dalloc(&P->psi[a][s][0], (size_t)P->psi_elems[a] * nshots * P->esize);
-            if (!st) st = dalloc(&P->psi[a][s][1], (size_t)P->psi_elems[a] * nshots * P->esize);
-            if (!st) st = dalloc(&P->xi[a][s], (size_t)P->xi_elems[a] * nshots * P->esize);
+        for (int s = 0; s < 2; ++s) {
+            L.add(&P->psi[a][s][0], (size_t)P->psi_elems[a] * nshots * P->esize);
+            L.add(&P->psi[a][s][1], (size_t)P->psi_elems[a] * nshots * P->esize);
+            L.add(&P->xi[a][s], (size_t)P->xi_elems[a] * nshots * P->esize);
         }
-        for (int c = 0; c < 8 && !st; ++c) st = dalloc(&P->coef[a][c], (size_t)(halo + 1) * P->esize);
     }
+    P->state_bytes = L.total;
+    const int64_t tiles = (nx + awcpml::kTileX - 1) / awcpml::kTileX;
+    P->fe_elems = ndim == 3 ? nz * tiles * 2 * ny : ny * tiles * 2;
+    L.add(&P->fact, (size_t)P->field_elems * P->esize);
+    L.add(&P->fact_edge, (size_t)P->fe_elems * P->esize);
+    for (int a = 0; a < ndim; ++a) L.add(&P->coef[a][0], (size_t)8 * (halo + 1) * P->esize);
+    st = group_alloc(P->main, L);
+    for (int a = 0; a < ndim && !st; ++a)
+        for (int c = 1; c < 8; ++c) P->coef[a][c] = (char*)P->coef[a][0] + (size_t)c * (halo + 1) * P->esize;
     if (!st) {
         hipError_t e = hipMemsetAsync(P->fact, 0, (size_t)P->field_elems * P->esize, P->stream);
         if (e == hipSuccess)
@@ -1667,28 +1730,28 @@ int awcpml_plan_destroy(awcpml_plan* P) {
     if (!P) return AWCPML_OK;
     if (P->stream) (void)hipStreamSynchronize(P->stream);
     drop_graphs(P->graphs);
-    for (int b = 0; b < 3; ++b) dfree(P->p[b]);
-    dfree(P->p_spare);
-    dfree(P->fact);
-    dfree(P->fact_edge);
+    // each buffer of its own, whatever role it plays now, then the groups
+    auto drop = [&](void*& v) {
+        if (!P->main.holds(v) && !P->spares.holds(v)) dfree(v);
+        v = nullptr;
+    };
+    for (int b = 0; b < 3; ++b) drop(P->p[b]);
+    drop(P->p_spare);
+    drop(P->fact);
+    drop(P->fact_edge);
     for (int a = 0; a < 3; ++a) {
         for (int s = 0; s < 2; ++s) {
-            dfree(P->psi[a][s][0]);
-            dfree(P->psi[a][s][1]);
-            dfree(P->psi_spare[a][s]);
-            dfree(P->xi[a][s]);
-            dfree(P->xi_spare[a][s]);
+            drop(P->psi[a][s][0]);
+            drop(P->psi[a][s][1]);
+            drop(P->psi_spare[a][s]);
+            drop(P->xi[a][s]);
+            drop(P->xi_spare[a][s]);
         }
-        for (int c = 0; c < 8; ++c) dfree(P->coef[a][c]);
+        drop(P->coef[a][0]);
     }
-    dfree(P->d_src_lin);
-    dfree(P->d_src_wav);
-    dfree(P->d_src_start);
-    dfree(P->d_src_seq);
-    dfree(P->d_rec_lin);
-    dfree(P->d_rec_start);
-    dfree(P->d_traces);
-    dfree(P->d_tile_io);
+    dfree(P->main.base);
+    dfree(P->spares.base);
+    io_free(P);
     dfree(P->ck);
     if (P->stage) (void)hipFree(P->stage);
     if (P->stream) (void)hipStreamDestroy(P->stream);
@@ -1734,11 +1797,13 @@ int awcpml_set_cpml(awcpml_plan* P, int axis, const double* a_l, const double* a
     if (axis < 0 || axis >= P->ndim) return fail(AWCPML_ERR_ARG, "axis %d out of range", axis);
     const double* v[8] = {a_l, a_r, b_K_l, b_K_r, a_hl, a_hr, b_K_hl, b_K_hr};
     const int h = P->halo;
+    std::vector<double> all((size_t)8 * (h + 1), 0.0);  // as the device holds them
     for (int c = 0; c < 8; ++c) {
         const size_t len = (size_t)h + (c >= 4 ? 1 : 0);
         if (len && !v[c]) return fail(AWCPML_ERR_ARG, "coefficient vector %d is NULL", c);
-        if ((st = upload(P, P->coef[axis][c], v[c], len))) return st;
+        if (len) memcpy(all.data() + (size_t)c * (h + 1), v[c], len * 8);
     }
+    if ((st = upload(P, P->coef[axis][0], all.data(), all.size()))) return st;
     HIP_TRY(hipStreamSynchronize(P->stream));
     for (int s = 0; s < 2; ++s) {
         bool idle = true;
@@ -1801,17 +1866,26 @@ int awcpml_reset(awcpml_plan* P) {
     if (st) return st;
     set_layout(P, P->home);
     const size_t fbytes = (size_t)P->field_elems * P->nshots * P->esize;
-    for (int b = 0; b < 3; ++b) HIP_TRY(hipMemsetAsync(P->p[b], 0, fbytes, P->stream));
-    if (P->p_spare) HIP_TRY(hipMemsetAsync(P->p_spare, 0, fbytes, P->stream));
+    // Buffers change places with the spares: cleared by block only where both
+    // sets lie in one each.
+    const bool one = P->main.base && (!P->p_spare || P->spares.base), two = one && P->spares.base;
+    if (one) HIP_TRY(hipMemsetAsync(P->main.base, 0, P->state_bytes, P->stream));
+    if (two) HIP_TRY(hipMemsetAsync(P->spares.base, 0, P->spares.bytes, P->stream));
+    for (int b = 0; b < 3 && !one; ++b) HIP_TRY(hipMemsetAsync(P->p[b], 0, fbytes, P->stream));
+    if (P->p_spare && !two) HIP_TRY(hipMemsetAsync(P->p_spare, 0, fbytes, P->stream));
     for (int a = 0; a < P->ndim; ++a)
         for (int s = 0; s < 2; ++s) {
             const size_t pb = (size_t)P->psi_elems[a] * P->nshots * P->esize;
             const size_t xb = (size_t)P->xi_elems[a] * P->nshots * P->esize;
-            HIP_TRY(hipMemsetAsync(P->psi[a][s][0], 0, pb, P->stream));
-            HIP_TRY(hipMemsetAsync(P->psi[a][s][1], 0, pb, P->stream));
-            if (P->psi_spare[a][s]) HIP_TRY(hipMemsetAsync(P->psi_spare[a][s], 0, pb, P->stream));
-            if (xb) HIP_TRY(hipMemsetAsync(P->xi[a][s], 0, xb, P->stream));
-            if (xb && P->xi_spare[a][s]) HIP_TRY(hipMemsetAsync(P->xi_spare[a][s], 0, xb, P->stream));
+            if (!one) {
+                HIP_TRY(hipMemsetAsync(P->psi[a][s][0], 0, pb, P->stream));
+                HIP_TRY(hipMemsetAsync(P->psi[a][s][1], 0, pb, P->stream));
+                if (xb) HIP_TRY(hipMemsetAsync(P->xi[a][s], 0, xb, P->stream));
+            }
+            if (!two && P->p_spare) {
+                HIP_TRY(hipMemsetAsync(P->psi_spare[a][s], 0, pb, P->stream));
+                if (xb) HIP_TRY(hipMemsetAsync(P->xi_spare[a][s], 0, xb, P->stream));
+            }
         }
     P->boundary_dirty = false;
     if (P->d_traces && P->n_rec_total > 0 && P->nt > 0)
@@ -2484,6 +2558,7 @@ struct AdjBuffers {
     void* grad = nullptr;
     void* grad64 = nullptr;
     void* tbar = nullptr;
+    void* list_block = nullptr;  // the lists below, packed
     void* node_lin = nullptr;
     void* node_start = nullptr;
     void* rec_start = nullptr;
@@ -2492,26 +2567,11 @@ struct AdjBuffers {
     void* rf_lin = nullptr;    // distinct receiver nodes over all shots
     void* rf_start = nullptr;  // CSR offsets into rf_idx
     void* rf_idx = nullptr;    // entries of each distinct node, in shot order
+    BufferGroup main, lists;   // all of them, in two groups
+    GroupList want_main, want_lists;
     ~AdjBuffers() {
-        for (auto& v : lam) dfree(v);
-        for (int a = 0; a < 3; ++a)
-            for (int s = 0; s < 2; ++s)
-                for (int b = 0; b < 2; ++b) {
-                    dfree(al[a][s][b]);
-                    dfree(be[a][s][b]);
-                }
-        dfree(q);
-        dfree(grad);
-        dfree(grad64);
-        dfree(tbar);
-        dfree(node_lin);
-        dfree(node_start);
-        dfree(rec_start);
-        dfree(rec_idx);
-        dfree(rq);
-        dfree(rf_lin);
-        dfree(rf_start);
-        dfree(rf_idx);
+        group_free(main, want_main);
+        group_free(lists, want_lists);
     }
 };
 
@@ -2578,33 +2638,34 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     const size_t fb = (size_t)P->field_elems * P->nshots * sizeof(T);
     AdjBuffers Bf;
     int st;
-    for (int b = 0; b < 3; ++b) {
-        if ((st = dalloc(&Bf.lam[b], fb))) return st;
-        HIP_TRY(hipMemsetAsync(Bf.lam[b], 0, fb, P->stream));
-    }
-    for (int a = 0; a < P->ndim; ++a)
-        for (int s = 0; s < 2; ++s)
-            for (int b = 0; b < 2; ++b) {
-                const size_t pb = (size_t)P->psi_elems[a] * P->nshots * sizeof(T);
-                const size_t xb = (size_t)P->xi_elems[a] * P->nshots * sizeof(T);
-                if ((st = dalloc(&Bf.al[a][s][b], pb))) return st;
-                if ((st = dalloc(&Bf.be[a][s][b], xb))) return st;
-                HIP_TRY(hipMemsetAsync(Bf.al[a][s][b], 0, pb, P->stream));
-                if (xb) HIP_TRY(hipMemsetAsync(Bf.be[a][s][b], 0, xb, P->stream));
-            }
-    if ((st = dalloc(&Bf.q, fb * (size_t)K))) return st;
     const AdjShape shape = adj_shape(P);
     if ((uint64_t)shape.blocks_per_group * shape.ngroups_cp > (uint64_t)INT32_MAX)
         return fail(AWCPML_ERR_ARG, "grid too large for the reverse step");
     const size_t gb = (size_t)P->field_elems * shape.ngroups_cp * sizeof(T);
-    if ((st = dalloc(&Bf.grad, gb))) return st;
-    HIP_TRY(hipMemsetAsync(Bf.grad, 0, gb, P->stream));
     const bool fold = P->grad_fold >= 0;
     const int64_t fold_every = P->grad_fold > 0 ? P->grad_fold : K;
     const int64_t nb_fold = (P->field_elems + 255) / 256;
-    if (fold) {
-        if ((st = dalloc(&Bf.grad64, (size_t)P->field_elems * 8))) return st;
-        HIP_TRY(hipMemsetAsync(Bf.grad64, 0, (size_t)P->field_elems * 8, P->stream));
+    const size_t ntr = (size_t)P->n_rec_total * nt;
+    // what starts as zeros, then q and the trace cotangents
+    GroupList& L = Bf.want_main;
+    for (int b = 0; b < 3; ++b) L.add(&Bf.lam[b], fb);
+    for (int a = 0; a < P->ndim; ++a)
+        for (int s = 0; s < 2; ++s)
+            for (int b = 0; b < 2; ++b) {
+                L.add(&Bf.al[a][s][b], (size_t)P->psi_elems[a] * P->nshots * sizeof(T));
+                L.add(&Bf.be[a][s][b], (size_t)P->xi_elems[a] * P->nshots * sizeof(T));
+            }
+    L.add(&Bf.grad, gb);
+    if (fold) L.add(&Bf.grad64, (size_t)P->field_elems * 8);
+    const size_t zeros = L.want.size(), zero_bytes = L.total;
+    L.add(&Bf.q, fb * (size_t)K);
+    L.add(&Bf.tbar, ntr * sizeof(T));
+    if ((st = group_alloc(Bf.main, L))) return st;
+    if (Bf.main.base) {
+        HIP_TRY(hipMemsetAsync(Bf.main.base, 0, zero_bytes, P->stream));
+    } else {
+        for (size_t q = 0; q < zeros; ++q)
+            if (L.want[q].second) HIP_TRY(hipMemsetAsync(*L.want[q].first, 0, L.want[q].second, P->stream));
     }
     int rf_count = 0;  // distinct receiver nodes (set below)
     auto fold_rq = [&](auto* total) -> int {
@@ -2623,8 +2684,6 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     };
 
     // trace cotangents and the distinct interior receiver nodes per shot
-    const size_t ntr = (size_t)P->n_rec_total * nt;
-    if ((st = dalloc(&Bf.tbar, ntr * sizeof(T)))) return st;
     if ((st = upload(P, Bf.tbar, tbar, ntr))) return st;
     std::vector<int64_t> node_lin;
     std::vector<int> node_start(1, 0), rec_start(1, 0), rec_idx;
@@ -2654,16 +2713,6 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         if (!v.empty()) rec_start.push_back((int)rec_idx.size());
         node_start.push_back((int)node_lin.size());
     }
-    if ((st = dalloc(&Bf.node_lin, node_lin.size() * 8))) return st;
-    if ((st = dalloc(&Bf.node_start, node_start.size() * 4))) return st;
-    if ((st = dalloc(&Bf.rec_start, rec_start.size() * 4))) return st;
-    if ((st = dalloc(&Bf.rec_idx, rec_idx.size() * 4))) return st;
-    if (!node_lin.empty()) {
-        HIP_TRY(hipMemcpyAsync(Bf.node_lin, node_lin.data(), node_lin.size() * 8, hipMemcpyHostToDevice, P->stream));
-        HIP_TRY(hipMemcpyAsync(Bf.rec_idx, rec_idx.data(), rec_idx.size() * 4, hipMemcpyHostToDevice, P->stream));
-    }
-    HIP_TRY(hipMemcpyAsync(Bf.node_start, node_start.data(), node_start.size() * 4, hipMemcpyHostToDevice, P->stream));
-    HIP_TRY(hipMemcpyAsync(Bf.rec_start, rec_start.data(), rec_start.size() * 4, hipMemcpyHostToDevice, P->stream));
     // the receiver gradient terms: one accumulator per entry of node_lin,
     // folded per distinct node over all shots in shot order
     std::vector<int64_t> rf_lin;
@@ -2683,15 +2732,28 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         if (!v.empty()) rf_start.push_back((int)rf_idx.size());
     }
     rf_count = (int)rf_lin.size();
-    if (rf_count) {
-        if ((st = dalloc(&Bf.rq, node_lin.size() * sizeof(T)))) return st;
-        HIP_TRY(hipMemsetAsync(Bf.rq, 0, node_lin.size() * sizeof(T), P->stream));
-        if ((st = dalloc(&Bf.rf_lin, rf_lin.size() * 8))) return st;
-        if ((st = dalloc(&Bf.rf_start, rf_start.size() * 4))) return st;
-        if ((st = dalloc(&Bf.rf_idx, rf_idx.size() * 4))) return st;
-        HIP_TRY(hipMemcpyAsync(Bf.rf_lin, rf_lin.data(), rf_lin.size() * 8, hipMemcpyHostToDevice, P->stream));
-        HIP_TRY(hipMemcpyAsync(Bf.rf_start, rf_start.data(), rf_start.size() * 4, hipMemcpyHostToDevice, P->stream));
-        HIP_TRY(hipMemcpyAsync(Bf.rf_idx, rf_idx.data(), rf_idx.size() * 4, hipMemcpyHostToDevice, P->stream));
+    {
+        std::vector<char> lists;
+        std::vector<std::pair<void**, size_t>> at;
+        auto put = [&](void** dst, const void* v, size_t bytes) {
+            at.push_back({dst, lists.size()});
+            lists.resize(lists.size() + (bytes + 7) / 8 * 8);
+            if (bytes) memcpy(lists.data() + at.back().second, v, bytes);
+        };
+        put(&Bf.node_lin, node_lin.data(), node_lin.size() * 8);
+        put(&Bf.rf_lin, rf_lin.data(), rf_lin.size() * 8);
+        put(&Bf.node_start, node_start.data(), node_start.size() * 4);
+        put(&Bf.rec_start, rec_start.data(), rec_start.size() * 4);
+        put(&Bf.rec_idx, rec_idx.data(), rec_idx.size() * 4);
+        put(&Bf.rf_start, rf_start.data(), rf_start.size() * 4);
+        put(&Bf.rf_idx, rf_idx.data(), rf_idx.size() * 4);
+        Bf.want_lists.add(&Bf.list_block, lists.size());
+        Bf.want_lists.add(&Bf.rq, node_lin.size() * sizeof(T));
+        if ((st = group_alloc(Bf.lists, Bf.want_lists))) return st;
+        for (auto& a : at) *a.first = (char*)Bf.list_block + a.second;
+        HIP_TRY(hipMemcpyAsync(Bf.list_block, lists.data(), lists.size(), hipMemcpyHostToDevice, P->stream));
+        if (rf_count) HIP_TRY(hipMemsetAsync(Bf.rq, 0, node_lin.size() * sizeof(T), P->stream));
+        HIP_TRY(hipStreamSynchronize(P->stream));  // `lists` leaves scope
     }
 
     awcpml::AdjIoArgs<T> io;
