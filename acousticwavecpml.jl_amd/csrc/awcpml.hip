@@ -21,6 +21,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -200,6 +201,8 @@ struct awcpml_plan {
     bool tb_auto = true;             // awcpml_set_time_block was not called: the library decides
     bool spare_failed = false;       // ... and the spare buffers did not fit
     int tb_rows = 0, tb_march = 0;   // waves per block, chunk length (0: default)
+    // 3D: two_shape's choice for the current CPML sides and tb_rows; 0: none yet
+    mutable int two_rows = 0, two_march = 0;
     int tb_prefetch = 0;             // planes of loads in flight (0: default)
     int tb_align = 1;                // 3D: aligned 64-lane tiles where no CPML slab reaches (FP32 default)
     void* p_spare = nullptr;
@@ -732,18 +735,23 @@ int do_step(awcpml_plan* P, int64_t it0) {
     return AWCPML_OK;
 }
 
-// Launches of several steps can run: spare buffers allocated, every field
+// Launches of several steps can run, given the spare buffers: every field
 // buffer zero on the Dirichlet nodes, at most kMaxSrc2 sources per shot, and
 // 32-bit byte offsets.  two_applies: two-step launches, which also write
 // d(pnew)/d(fact) only of both steps; two_ok: ... and were requested.
-bool multi_applies(const awcpml_plan* P) {
-    return P->p_spare && !P->src_on_boundary && P->src_per_shot_max <= awcpml::kMaxSrc2 &&
+bool multi_possible(const awcpml_plan* P) {
+    return !P->src_on_boundary && P->src_per_shot_max <= awcpml::kMaxSrc2 &&
            !P->boundary_dirty && !P->wide && (uint64_t)P->field_elems * P->esize < (1ull << 32);
 }
 
+bool multi_applies(const awcpml_plan* P) { return P->p_spare && multi_possible(P); }
+
 bool two_applies(const awcpml_plan* P) { return multi_applies(P) && (!P->q_cur || P->q_next); }
 
-bool two_ok(const awcpml_plan* P) { return P->time_block == 2 && two_applies(P); }
+// (3D; a plan left to the library's choice takes them too)
+bool two_ok(const awcpml_plan* P) {
+    return (P->time_block == 2 || (P->tb_auto && P->ndim == 3)) && two_applies(P);
+}
 
 // A 2D plan takes the tile kernel: by the library's own choice, or where
 // two-step launches were requested.
@@ -753,7 +761,8 @@ bool tile_ok(const awcpml_plan* P) {
 
 int two_rows_default(int ndim, int dtype) { return ndim == 2 ? 4 : (dtype == AWCPML_F64 ? 8 : 16); }
 
-// The plan's chunk length of two-step launches with W waves per block.
+// The chunk length of a plan's share of two-step batch launches (W waves per
+// block), and of 3D plans where it is set.
 int two_march(const awcpml_plan* P, int W) {
     if (P->tb_march > 0) return P->tb_march;
     if (P->ndim == 2) return (int)std::max<int64_t>(8, std::min<int64_t>(64, (P->n[1] - 2) / 16));
@@ -763,13 +772,6 @@ int two_march(const awcpml_plan* P, int W) {
     const int64_t interior = P->n[2] - 2;
     const int64_t want = std::max<int64_t>(1, (2048 + tiles - 1) / tiles);
     return (int)std::max<int64_t>(16, std::min<int64_t>((interior + want - 1) / want, 128));
-}
-
-void two_tiling(const awcpml_plan* P, int* rows, int* march, int* prefetch) {
-    const int W = P->tb_rows > 0 ? P->tb_rows : two_rows_default(P->ndim, P->dtype);
-    *rows = W;
-    *march = two_march(P, W);
-    *prefetch = P->tb_prefetch > 0 ? P->tb_prefetch : 2;
 }
 
 // March chunks of a two-step launch (chunk_start[0..count]), or 0 for
@@ -797,6 +799,87 @@ int two_chunk_list(const awcpml_plan* P, int ml, int* starts) {
         for (int64_t q = 1; q <= pieces; ++q) starts[++count] = (int)(b0 + (b1 - b0) * q / pieces);
     }
     return count;
+}
+
+// Waves per block and chunk length of a 3D plan's two-step launches where they
+// are not set: the shape whose slowest XCD is done first.  An XCD works through
+// an eighth of the blocks in order (x, y tiles, then chunks, then shots) on 32
+// CUs; a block's time is its planes (1.3 times in the CPML layers) and 20 (FP32:
+// 16) more for its start and the planes at its ends.  FP64 blocks of 8 waves and
+// FP32 blocks of 16 have a CU to themselves; two FP32 blocks of 8 share one and
+// are 5 % faster for their rows.  Up to 256 blocks are placed one by one, more
+// take their mean and half a block.  FP64 chunks stay below 49 planes: blocks
+// that march further drift apart and find less in L2 (450x430x300: 461 us per
+// step at 40 planes, 534 at 96; 298^3, 3 shots: 627 and 718), unless whole shots
+// or halves of them share out evenly among the XCDs (298^3, 4 shots: 816 and
+// 785; 200x180x190, 8 shots: 560 and 539).
+// On 39 grids and shot counts from 30x32x28 to 450x430x300 nodes, every shape
+// timed, this is 1.4 % above the best shape on average and 19 % at worst; 2048
+// blocks of 16 to 128 planes, the rule of batches, are up to 40 % above it.
+void two_shape(const awcpml_plan* P, int* rows, int* march) {
+    const bool f64 = P->dtype == AWCPML_F64;
+    const bool slabs = P->halo > 0 && (P->active[2][0] || P->active[2][1]);
+    double best = 0;
+    for (int W : {16, 8, 4}) {
+        if (P->tb_rows > 0 ? W != P->tb_rows : (W == 4 || (f64 && W == 16))) continue;
+        const int64_t tiles = ((P->n[0] - 2 + awcpml::kOwnX - 1) / awcpml::kOwnX) *
+                              ((P->n[1] - 2 + W - 3) / (W - 2));
+        const int share = std::max(1, (f64 ? 8 : 16) / W);  // blocks on a CU together
+        const size_t slots = (size_t)32 * share;
+        for (int ml : {4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 36, 40, 48, 56, 64, 80, 96}) {
+            if (f64 && ml > 48 && P->nshots % 4 != 0) break;
+            int starts[awcpml::kMaxChunks2 + 1];
+            int64_t n = two_chunk_list(P, ml, starts);
+            const bool uniform = n == 0;
+            if (uniform) n = (P->n[2] - 2 + ml - 1) / ml;
+            auto block_time = [&](int64_t c) {
+                const int64_t z0 = uniform ? 1 + c * ml : starts[c];
+                const int64_t z1 = uniform ? std::min<int64_t>(z0 + ml, P->n[2] - 1) : starts[c + 1];
+                const bool layer = slabs && (uniform || (P->active[2][0] && z1 <= P->halo + 2) ||
+                                             (P->active[2][1] && z0 >= P->n[2] - P->halo - 2));
+                return (f64 ? 20 : 16) + (layer ? 1.3 : 1.0) * (double)(z1 - z0);
+            };
+            const int64_t total = tiles * n * P->nshots;
+            const int64_t per = (total + awcpml::kNumXcd - 1) / awcpml::kNumXcd;
+            double slowest = 0;
+            if (per > 256 * share) {
+                double sum = 0, longest = 0;
+                for (int64_t c = 0; c < n; ++c) {
+                    sum += block_time(c) / (double)n;
+                    longest = std::max(longest, block_time(c));
+                }
+                slowest = sum * (double)per / (double)slots + longest / 2;
+            } else {
+                for (int64_t x0 = 0; x0 < total; x0 += per) {
+                    std::vector<double> busy(slots, 0.0);  // a heap, first free on top
+                    for (int64_t q = x0; q < std::min(total, x0 + per); ++q) {
+                        std::pop_heap(busy.begin(), busy.end(), std::greater<>());
+                        busy.back() += block_time(q / tiles % n);
+                        slowest = std::max(slowest, busy.back());
+                        std::push_heap(busy.begin(), busy.end(), std::greater<>());
+                    }
+                }
+            }
+            if (!f64 && W == 8) slowest *= 0.95;
+            if (best == 0 || slowest < best) {
+                best = slowest;
+                *rows = W;
+                *march = ml;
+            }
+        }
+    }
+}
+
+void two_tiling(const awcpml_plan* P, int* rows, int* march, int* prefetch) {
+    if (P->ndim == 3 && P->tb_march == 0) {
+        if (P->two_march == 0) two_shape(P, &P->two_rows, &P->two_march);
+        *rows = P->two_rows;
+        *march = P->two_march;
+    } else {
+        *rows = P->tb_rows > 0 ? P->tb_rows : two_rows_default(P->ndim, P->dtype);
+        *march = two_march(P, *rows);
+    }
+    *prefetch = P->tb_prefetch > 0 ? P->tb_prefetch : 2;
 }
 
 // Aligned 64-lane tiles need the plain stencil at the nodes just outside
@@ -968,10 +1051,11 @@ void two_swap(awcpml_plan* P) {
 }
 
 template <typename T>
-int io_two_t(awcpml_plan* P, int64_t it0, int rot, bool inject) {
-    awcpml::IoArgs<T> A = make_io<T>(P, rot);
-    A.inject = inject ? 1 : 0;
-    awcpml::sources_receivers<T><<<dim3(P->nshots), dim3(256), 0, P->stream>>>(A, it0);
+int io_two_t(awcpml_plan* P, int64_t it0, int rot1, int rot2) {
+    awcpml::IoArgs<T> A1 = make_io<T>(P, rot1), A2 = make_io<T>(P, rot2);
+    A1.pnew = (T*)P->p[P->rot % 3];  // p^{t+1}: pold of the step to come
+    A1.inject = 0;
+    awcpml::sources_receivers_two<T><<<dim3(P->nshots), dim3(256), 0, P->stream>>>(A1, A2, it0);
     HIP_TRY(hipGetLastError());
     return AWCPML_OK;
 }
@@ -983,17 +1067,10 @@ int do_step2(awcpml_plan* P, int64_t it0) {
     const bool f64 = P->dtype == AWCPML_F64;
     int st = f64 ? launch_stencil2_t<double>(P, it0) : launch_stencil2_t<float>(P, it0);
     if (st) return st;
-    if (P->has_io) {
-        st = f64 ? io_two_t<double>(P, it0, P->rot, false) : io_two_t<float>(P, it0, P->rot, false);
-        if (st) return st;
-    }
-    const int rot1 = (P->rot + 1) % 3;
+    const int rot0 = P->rot, rot1 = (P->rot + 1) % 3;
     two_swap(P);
-    if (P->has_io) {
-        st = f64 ? io_two_t<double>(P, it0 + 1, rot1, true) : io_two_t<float>(P, it0 + 1, rot1, true);
-        if (st) return st;
-    }
-    return AWCPML_OK;
+    if (P->has_io) st = f64 ? io_two_t<double>(P, it0, rot0, rot1) : io_two_t<float>(P, it0, rot0, rot1);
+    return st;
 }
 
 int do_tile(awcpml_plan* P, int64_t it0, int steps, void* q) {
@@ -1144,10 +1221,25 @@ int alloc_spares(awcpml_plan* P) {
     return AWCPML_OK;
 }
 
+constexpr size_t kAskFreeBytes = 64ull << 20;
+
 // A plan left to the library's choice gets its spare buffers with its first
-// run of several steps; where they do not fit it keeps single steps.
+// run of several steps; where they do not fit, or would take more than an
+// eighth of the device memory that is free (which the caller may count on), it
+// keeps single steps.
 int auto_spares(awcpml_plan* P, int64_t n) {
-    if (!P->tb_auto || P->ndim != 2 || n < 2 || P->p_spare || P->spare_failed) return AWCPML_OK;
+    if (!P->tb_auto || n < 2 || P->p_spare || P->spare_failed || !multi_possible(P)) return AWCPML_OK;
+    int64_t elems = P->field_elems;
+    for (int a = 0; a < P->ndim; ++a) elems += 2 * (P->psi_elems[a] + P->xi_elems[a]);
+    const size_t bytes = (size_t)elems * P->nshots * P->esize;
+    size_t avail = 0, total = 0;
+    if (bytes > kAskFreeBytes) {
+        HIP_TRY(hipMemGetInfo(&avail, &total));
+        if (bytes > avail / 8) {
+            P->spare_failed = true;
+            return AWCPML_OK;
+        }
+    }
     const int st = alloc_spares(P);
     if (st != AWCPML_ERR_NOMEM) return st;
     (void)hipGetLastError();
@@ -1812,6 +1904,7 @@ int awcpml_set_cpml(awcpml_plan* P, int axis, const double* a_l, const double* a
         P->active[axis][s] = (h > 0 && !idle) ? 1 : 0;
     }
     P->cpml_set[axis] = true;
+    P->two_march = 0;
     P->ck_valid = false;
     drop_graphs(P->graphs);
     ++P->gen;
@@ -2081,6 +2174,7 @@ int awcpml_set_time_block(awcpml_plan* P, int steps, int block_rows, int march_l
     P->tb_rows = block_rows;
     P->tb_march = march_len;
     P->tb_prefetch = prefetch;
+    P->two_march = 0;
     drop_graphs(P->graphs);
     ++P->gen;
     return AWCPML_OK;

@@ -930,6 +930,16 @@ __global__ __launch_bounds__(256) void sources_receivers(const IoArgs<T> A, int6
     io_block(A, blockIdx.x, it0);
 }
 
+// A two-step launch's pair: step it0's receivers (its sources are already in
+// A1's field), then step it0+1's sources and receivers in A2's.  One launch of
+// latency instead of two (about 1.5 us per step).
+template <typename T>
+__global__ __launch_bounds__(256) void sources_receivers_two(const IoArgs<T> A1, const IoArgs<T> A2,
+                                                             int64_t it0) {
+    io_block(A1, blockIdx.x, it0);
+    io_block(A2, blockIdx.x, it0 + 1);
+}
+
 // Batch: block b serves shot b - shot_start[p] of plan p.
 template <typename T>
 struct IoBatchArgs {

@@ -167,9 +167,8 @@ int awcpml_get_shot_group(const awcpml_plan *plan, int *shot_group);
  * reset, whose pressure there must rotate through the three field buffers
  * exactly as the reference's does).  Results are bit-identical to one step
  * per launch.  steps = 1: one step per launch.  A plan for which this is
- * never called chooses by itself: 2D plans take launches of several steps
- * where those apply and their spare buffers fit (allocated with the first
- * run of two steps or more), 3D plans single steps.
+ * never called takes launches of several steps where those apply and their
+ * spare buffers fit (allocated with the first run of two steps or more).
  * 3D launch shape: block_rows is the number of wavefronts per block, 4, 8
  * or 16 (the block updates block_rows-2 rows and recomputes the first step
  * on the two outer ones), march_len the chunk along z, prefetch the planes
