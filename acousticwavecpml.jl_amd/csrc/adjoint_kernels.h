@@ -67,16 +67,17 @@ struct AdjointArgs {
     int64_t xi_stride[3];
     int ndim;
     int nshots;
-    int group;                // shots per thread (one gradient accumulator per group)
+    int group[2];             // shots per thread (one gradient accumulator per group)
+                              // outside and in the block classes with CPML nodes
     int tiles_x, tiles_y;     // 64-wide x tiles, row groups
     // block classes: per axis (x tiles, row groups, 3D planes) the tiles
     // none of whose nodes lies in the CPML range of an absorbing side,
     // [int_lo, int_hi) of ntiles; class c (bit a set: the tiles of axis a
-    // outside that range) holds the launch's logical blocks
-    // [cls_start[c], cls_start[c+1])
+    // outside that range).  Class 0 has blocks[0] blocks, classes 1 and up
+    // blocks[1], class c from cls_start[c] on
     int ntiles[3], int_lo[3], int_hi[3];
     int cls_start[9];
-    int logical_blocks, grid_blocks;
+    int blocks[2];
 };
 
 // Element index of layer L of axis a's slab at node (i, j, k) in a slab
@@ -103,13 +104,25 @@ struct AdjCoef {
     T bKh_hi, ah_hi;   // edge m
 };
 
+// Layers m-2, m-1, m of 0..h-1 and edges m-1, m of 0..h, clamped so that every
+// lane may load them; a value counts only where its flag in AdjCoef is set.
+struct AdjLayers {
+    int b0, b1, b2, lo, hi;
+};
+
+__device__ __forceinline__ AdjLayers adj_layers(int m, int h) {
+    AdjLayers L;
+    L.b0 = min(max(m - 2, 0), h - 1);
+    L.b1 = min(max(m - 1, 0), h - 1);
+    L.b2 = min(m, h - 1);
+    L.lo = min(max(m - 1, 0), h);
+    L.hi = min(m, h);
+    return L;
+}
+
 template <typename T>
-__device__ __forceinline__ AdjCoef<T> adj_coef(const AdjointArgs<T>& A, int a, int64_t c) {
+__device__ __forceinline__ AdjCoef<T> adj_coef(const AdjointArgs<T>& A, int a, int64_t c, AdjLayers& L) {
     AdjCoef<T> C;
-    C.ext = C.v0 = C.v1 = C.v2 = C.e_lo = C.e_hi = C.w_lo = false;
-    C.side = 0;
-    C.m = 0;
-    C.a0 = C.a1 = C.a2 = C.bK1 = C.bKh_lo = C.ah_lo = C.bKh_hi = C.ah_hi = T(0);
     const int64_t h = A.halo;
     int64_t m = -1;
     int side = 0;
@@ -119,34 +132,28 @@ __device__ __forceinline__ AdjCoef<T> adj_coef(const AdjointArgs<T>& A, int a, i
         m = c - (A.n[a] - h - 2);
         side = 1;
     }
-    if (m < 0 || m > h + 1) return C;
+    C.ext = m >= 0 && m <= h + 1;
+    C.side = side;
+    C.m = C.ext ? (int)m : 0;
+    L = adj_layers(C.m, (int)h);
     const T* av = side ? A.side[a][1].a : A.side[a][0].a;
     const T* bK = side ? A.side[a][1].bK : A.side[a][0].bK;
     const T* bKh = side ? A.side[a][1].bKh : A.side[a][0].bKh;
     const T* ah = side ? A.side[a][1].ah : A.side[a][0].ah;
-    C.ext = true;
-    C.side = side;
-    C.m = (int)m;
-    C.v0 = m >= 2 && m - 1 <= h;
-    C.v1 = m >= 1 && m <= h;
-    C.v2 = m + 1 <= h;
-    if (C.v0) C.a0 = av[m - 2];
-    if (C.v1) {
-        C.a1 = av[m - 1];
-        C.bK1 = bK[m - 1];
-    }
-    if (C.v2) C.a2 = av[m];
-    C.e_lo = m >= 1;
-    C.e_hi = m <= h;
-    C.w_lo = m == 1 && side == 0;
-    if (C.e_lo) {
-        C.bKh_lo = bKh[m - 1];
-        C.ah_lo = ah[m - 1];
-    }
-    if (C.e_hi) {
-        C.bKh_hi = bKh[m];
-        C.ah_hi = ah[m];
-    }
+    C.a0 = av[L.b0];
+    C.a1 = av[L.b1];
+    C.a2 = av[L.b2];
+    C.bK1 = bK[L.b1];
+    C.bKh_lo = bKh[L.lo];
+    C.ah_lo = ah[L.lo];
+    C.bKh_hi = bKh[L.hi];
+    C.ah_hi = ah[L.hi];
+    C.v0 = C.ext && m >= 2 && m - 1 <= h;
+    C.v1 = C.ext && m >= 1 && m <= h;
+    C.v2 = C.ext && m + 1 <= h;
+    C.e_lo = C.ext && m >= 1;
+    C.e_hi = C.ext && m <= h;
+    C.w_lo = C.ext && m == 1 && side == 0;
     return C;
 }
 
@@ -157,24 +164,12 @@ struct AdjVals {
     T b0, b1, b2, alo, ahi;
 };
 
-// ob: offset of the node's own beta (layer m); oa: offset of alpha edge
-// m-1; ls: offset between neighbouring layers/edges.
-template <typename T>
-__device__ __forceinline__ void adj_vals(const AdjCoef<T>& C, const T* be, const T* al,
-                                         int64_t ob, int64_t oa, int64_t ls, AdjVals<T>& V) {
-    V.b0 = C.v0 ? be[ob - ls] : T(0);
-    V.b1 = C.v1 ? be[ob] : T(0);
-    V.b2 = C.v2 ? be[ob + ls] : T(0);
-    V.alo = C.e_lo ? al[oa] : T(0);
-    V.ahi = C.e_hi ? al[oa + ls] : T(0);
-}
-
-// One axis's slab terms of lam^s (added to acc) and its alpha^{s+1} stores.
+// One axis's slab terms of lam^s (added to acc) and its alpha^{s+1} stores
+// (alo, ahi: where edges m-1 and m are kept).
 // um/uc/up: f lam^{s+1} one node below, at and above the node on the axis.
 template <typename T>
 __device__ __forceinline__ void adj_term(const AdjCoef<T>& C, const AdjVals<T>& V, T um, T uc,
-                                         T up, T inv_d, T inv_d2, T* alw, int64_t oa,
-                                         int64_t ls, T& acc) {
+                                         T up, T inv_d, T inv_d2, T* alo, T* ahi, T& acc) {
     const T z0 = C.v0 ? C.a0 * V.b0 : T(0);
     const T z1 = C.v1 ? C.a1 * V.b1 : T(0);
     const T z2 = C.v2 ? C.a2 * V.b2 : T(0);
@@ -185,84 +180,57 @@ __device__ __forceinline__ void adj_term(const AdjCoef<T>& C, const AdjVals<T>& 
     if (C.e_lo) {
         const T alv = C.bKh_lo * V.alo + (w0 - w1) * inv_d;
         y_lo = C.ah_lo * alv;
-        if (C.w_lo) alw[oa] = alv;
+        if (C.w_lo) *alo = alv;
     }
     if (C.e_hi) {
         const T alv = C.bKh_hi * V.ahi + (w1 - w2) * inv_d;
         y_hi = C.ah_hi * alv;
-        alw[oa + ls] = alv;
+        *ahi = alv;
     }
     acc += (y_lo - y_hi) * inv_d;
     acc += (z0 - T(2) * z1 + z2) * inv_d2;
 }
 
-// CPML data of one node on one axis with its slab offsets: ob of the
-// node's own beta layer m-1, oa of alpha edge m-1, ls between neighbouring
-// layers/edges (offsets follow slab_index).
-template <typename T>
-struct AdjAxis {
-    AdjCoef<T> C;
-    int64_t ob, oa, ls;
-};
-
-template <typename T>
-__device__ __forceinline__ AdjAxis<T> adj_axis(const AdjointArgs<T>& A, int a, int64_t i,
-                                               int64_t j, int64_t k) {
-    AdjAxis<T> X;
-    const int64_t c = a == 0 ? i : (a == 1 ? j : k);
-    X.C = adj_coef<T>(A, a, c);
-    const int64_t h = A.halo, ny = A.n[1], px = A.px, L = X.C.m - 1;
-    X.ob = slab_index(a, h, L, i, j, k, px, ny);
-    X.oa = slab_index(a, h + 1, L, i, j, k, px, ny);
-    X.ls = a == 0 ? 1 : (a == 1 ? px : px * ny);
-    return X;
-}
-
-// Everything one shot reads at one node: lam^{s+1} at the node and its
-// axis neighbours, lam^{s+2}, q^s and (CP) the slab values of every axis
-// whose CPML range holds the node.
-template <typename T, int NDIM, bool CP>
+// Everything one shot reads at one node outside the CPML ranges: lam^{s+1} at
+// the node and its axis neighbours, lam^{s+2} and q^s.
+template <typename T, int NDIM>
 struct AdjShot {
     T lc, lm[NDIM], lp[NDIM], l2, q;
-    AdjVals<T> v[CP ? NDIM : 1];
 };
 
-template <typename T, int NDIM, bool CP>
-__device__ __forceinline__ void adj_load_shot(const AdjointArgs<T>& A, const AdjAxis<T>* X,
-                                              int g, int64_t lin, const int64_t* so,
-                                              AdjShot<T, NDIM, CP>& S) {
-    const int64_t fs = (int64_t)g * A.field_stride;
-    const T* l1 = A.lam1 + fs;
-    S.lc = l1[lin];
-#pragma unroll
-    for (int a = 0; a < NDIM; ++a) {
-        S.lm[a] = l1[lin - so[a]];
-        S.lp[a] = l1[lin + so[a]];
-    }
-    S.l2 = A.lam2[fs + lin];
-    S.q = A.q[fs + lin];
-    if constexpr (CP) {
-#pragma unroll
-        for (int a = 0; a < NDIM; ++a) {
-            if (!X[a].C.ext) continue;
-            const bool hi = X[a].C.side != 0;
-            const T* be = hi ? A.side[a][1].be_rd : A.side[a][0].be_rd;
-            const T* al = hi ? A.side[a][1].al_rd : A.side[a][0].al_rd;
-            adj_vals(X[a].C, be + g * A.xi_stride[a], al + g * A.psi_stride[a], X[a].ob,
-                     X[a].oa, X[a].ls, S.v[a]);
-        }
-    }
+// Value at byte offset o; the base is the same for all lanes of a wave, so the
+// load takes it from scalar registers and needs one offset register.
+template <typename T, typename Off>
+__device__ __forceinline__ T adj_at(const T* base, Off o) {
+    return *(const T*)((const char*)base + o);
 }
 
-// Shot g's reverse step at the node from its loads S: stores lam^s (and,
-// CP, the slab values) and returns lam^s q^s, the node's gradient term.
-template <typename T, int NDIM, bool CP>
-__device__ __forceinline__ T adj_shot(const AdjointArgs<T>& A, const AdjAxis<T>* X, int g,
-                                      int64_t lin, T fc, const T* fm, const T* fp,
-                                      const AdjShot<T, NDIM, CP>& S) {
+template <typename T, typename Off>
+__device__ __forceinline__ T* adj_ptr(T* base, Off o) {
+    return (T*)((char*)base + o);
+}
+
+// off: byte offset of the node
+template <typename T, int NDIM, typename Off>
+__device__ __forceinline__ void adj_load_shot(const AdjointArgs<T>& A, int g, Off off, const int64_t* so,
+                                              AdjShot<T, NDIM>& S) {
     const int64_t fs = (int64_t)g * A.field_stride;
-    const T uc = fc * S.lc;
-    T um[NDIM], up[NDIM];
+    const T* l1 = A.lam1 + fs;
+    S.lc = adj_at(l1, off);
+#pragma unroll
+    for (int a = 0; a < NDIM; ++a) {
+        S.lm[a] = adj_at(l1 - so[a], off);
+        S.lp[a] = adj_at(l1 + so[a], off);
+    }
+    S.l2 = adj_at(A.lam2 + fs, off);
+    S.q = adj_at(A.q + fs, off);
+}
+
+// The plain part of lam^s; um/uc/up: f lam^{s+1} around the node.
+template <typename T, int NDIM>
+__device__ __forceinline__ T adj_plain(const AdjointArgs<T>& A, T fc, const T* fm, const T* fp,
+                                       const AdjShot<T, NDIM>& S, T& uc, T* um, T* up) {
+    uc = fc * S.lc;
     T acc = T(2) * S.lc - S.l2;
 #pragma unroll
     for (int a = 0; a < NDIM; ++a) {
@@ -270,42 +238,24 @@ __device__ __forceinline__ T adj_shot(const AdjointArgs<T>& A, const AdjAxis<T>*
         up[a] = fp[a] * S.lp[a];
         acc += (up[a] - T(2) * uc + um[a]) * A.inv_d2[a];
     }
-    if constexpr (CP) {
-#pragma unroll
-        for (int a = 0; a < NDIM; ++a) {
-            if (!X[a].C.ext) continue;
-            T* alw = (X[a].C.side ? A.side[a][1].al_wr : A.side[a][0].al_wr) +
-                     g * A.psi_stride[a];
-            adj_term(X[a].C, S.v[a], um[a], uc, up[a], A.inv_d[a], A.inv_d2[a], alw, X[a].oa,
-                     X[a].ls, acc);
-        }
-    }
-    A.lam0[fs + lin] = acc;
-    if constexpr (CP) {
-        // beta^s = bK beta^{s+1} + f lam^s on every slab holding the node
-#pragma unroll
-        for (int a = 0; a < NDIM; ++a) {
-            if (!(X[a].C.ext && X[a].C.v1)) continue;
-            T* bew = (X[a].C.side ? A.side[a][1].be_wr : A.side[a][0].be_wr) +
-                     g * A.xi_stride[a];
-            bew[X[a].ob] = X[a].C.bK1 * S.v[a].b1 + fc * acc;
-        }
-    }
-    return acc * S.q;
+    return acc;
 }
 
 // One shot of the three-slot pipeline: refill slot F with shot g+2's
-// loads, then compute shot g from slot C (loaded two shots earlier).
-template <typename T, int NDIM, bool CP>
-__device__ __forceinline__ void adj_pipe(const AdjointArgs<T>& A, const AdjAxis<T>* X, int g,
-                                         int g1, int64_t lin, const int64_t* so, T fc,
-                                         const T* fm, const T* fp, AdjShot<T, NDIM, CP>& C,
-                                         AdjShot<T, NDIM, CP>& F, T& gsum) {
+// loads, then compute shot g from slot C (loaded two shots earlier): its
+// lam^s is stored, its gradient term lam^s q^s added to gsum.
+template <typename T, int NDIM, typename Off>
+__device__ __forceinline__ void adj_pipe(const AdjointArgs<T>& A, int g, int g1, Off off, const int64_t* so,
+                                         T fc, const T* fm, const T* fp, AdjShot<T, NDIM>& C,
+                                         AdjShot<T, NDIM>& F, T& gsum) {
     if (g >= g1) return;
-    if (g + 2 < g1) adj_load_shot<T, NDIM, CP>(A, X, g + 2, lin, so, F);
+    if (g + 2 < g1) adj_load_shot<T, NDIM>(A, g + 2, off, so, F);
     // keep the later shots' loads ahead of this shot's arithmetic
     __builtin_amdgcn_sched_barrier(0);
-    gsum += adj_shot<T, NDIM, CP>(A, X, g, lin, fc, fm, fp, C);
+    T uc, um[NDIM], up[NDIM];
+    const T acc = adj_plain<T, NDIM>(A, fc, fm, fp, C, uc, um, up);
+    *adj_ptr(A.lam0 + (int64_t)g * A.field_stride, off) = acc;
+    gsum += acc * C.q;
 }
 
 // Tiles of axis a in block class c, and the u-th of them.
@@ -317,70 +267,211 @@ __device__ __forceinline__ int adj_class_tile(int c, int lo, int hi, int a, int 
     return u < lo ? u : hi + (u - lo);
 }
 
-// One reverse step.  Block (64, BY): lane -> x, threadIdx.y -> y row; a
-// thread owns one interior node (plane k in 3D) and walks the shots of
-// its shot group, so fact, the CPML coefficients and the gradient
-// accumulator of the node are read once per group and the group's
-// gradient terms are summed in registers (one read-modify-write of the
-// group's accumulator per step).  Shots run through a three-slot pipeline:
-// the loads of shots g+1 and g+2 are in flight while shot g is computed.
-// CP = false: the launch covers block class 0 (no node of the block in a
-// CPML range) and carries no slab code, so it runs with the registers of
-// the plain stencil; CP = true: classes 1 and up.  Logical blocks within a
-// class: x tile fastest, then row group, plane (3D), shot group,
-// renumbered XCD-aware.
+// The node of a thread of a reverse step's launch.  Block (64, BY): lane -> x,
+// threadIdx.y -> y row, plane k in 3D; a thread owns one interior node and walks
+// the shots g0 .. g1-1 of its group.  Logical blocks within a class: x tile
+// fastest, then row group, plane (3D), shot group, renumbered XCD-aware.
+struct AdjNode {
+    int cls, grp, g0, g1;
+    int64_t i, j, k;
+};
+
+// lb: the block's number among those of class 0 (CP = false) or 1..7.
 template <typename T, int NDIM, bool CP>
-__global__ __launch_bounds__(256) void adjoint_step(const AdjointArgs<T> A) {
-    const int lb = logical_block(blockIdx.x, A.grid_blocks);
-    if (lb >= A.logical_blocks) return;
-    const int64_t nx = A.n[0], ny = A.n[1], px = A.px;
-    int cls = 0;
+__device__ __forceinline__ bool adj_node(const AdjointArgs<T>& A, int lb, AdjNode& N) {
+    if (lb >= A.blocks[CP]) return false;
+    N.cls = 0;
     if (CP)
         for (int c = 1; c < 8; ++c)
-            if (lb >= A.cls_start[c]) cls = c;
-    int rest = lb - A.cls_start[cls];
+            if (lb >= A.cls_start[c]) N.cls = c;
+    int rest = CP ? lb - A.cls_start[N.cls] : lb;
     int t[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const int na = adj_class_tiles(cls, A.ntiles[a], A.int_lo[a], A.int_hi[a], a);
-        t[a] = adj_class_tile(cls, A.int_lo[a], A.int_hi[a], a, rest % na);
+        const int na = adj_class_tiles(N.cls, A.ntiles[a], A.int_lo[a], A.int_hi[a], a);
+        t[a] = adj_class_tile(N.cls, A.int_lo[a], A.int_hi[a], a, rest % na);
         rest /= na;
     }
-    const int grp = rest;
-    const int64_t k = NDIM == 3 ? 1 + t[2] : 0;
-    const int64_t i = (int64_t)t[0] * kTileX + threadIdx.x;
+    N.grp = rest;
+    N.g0 = rest * A.group[CP];
+    N.g1 = N.g0 + A.group[CP] < A.nshots ? N.g0 + A.group[CP] : A.nshots;
+    N.k = NDIM == 3 ? 1 + t[2] : 0;
+    N.i = (int64_t)t[0] * kTileX + threadIdx.x;
     // one row per wavefront: j (and the y axis's CPML data) is wave-uniform
-    const int wy = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int64_t j = 1 + (int64_t)t[1] * blockDim.y + wy;
-    if (i < 1 || i > nx - 2 || j > ny - 2) return;
-    const int64_t so[3] = {1, px, px * ny};
-    const int64_t lin = i + px * j + so[2] * k;
+    N.j = 1 + (int64_t)t[1] * blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    return N.i >= 1 && N.i <= A.n[0] - 2 && N.j <= A.n[1] - 2;
+}
+
+// One reverse step of the nodes of block class 0 (no node of the block in a
+// CPML range).  fact and the gradient accumulator of the node are read once per
+// group of shots, whose gradient terms are summed in registers (one
+// read-modify-write of the group's accumulator per step).  Shots run through a
+// three-slot pipeline: the loads of shots g+1 and g+2 are in flight while shot g
+// is computed.
+template <typename T, int NDIM, typename Off>
+__device__ __forceinline__ void adj_plain_block(const AdjointArgs<T>& A, int lb) {
+    AdjNode N;
+    if (!adj_node<T, NDIM, false>(A, lb, N)) return;
+    const int64_t so[3] = {1, A.px, A.px * A.n[1]};
+    const Off off = (Off)((N.i + A.px * N.j + so[2] * N.k) * (int64_t)sizeof(T));
     const T* f = A.fact;
-    const T fc = f[lin];
+    const T fc = adj_at(f, off);
     T fm[NDIM], fp[NDIM];
 #pragma unroll
     for (int a = 0; a < NDIM; ++a) {
-        fm[a] = f[lin - so[a]];
-        fp[a] = f[lin + so[a]];
+        fm[a] = adj_at(f - so[a], off);
+        fp[a] = adj_at(f + so[a], off);
     }
-    AdjAxis<T> X[CP ? NDIM : 1];
-    if constexpr (CP) {
-#pragma unroll
-        for (int a = 0; a < NDIM; ++a) X[a] = adj_axis<T>(A, a, i, j, k);
-    }
-    const int g0 = grp * A.group;
-    const int g1 = g0 + A.group < A.nshots ? g0 + A.group : A.nshots;
+    const int g0 = N.g0, g1 = N.g1;
     T gsum = T(0);
-    AdjShot<T, NDIM, CP> s0, s1, s2;
-    adj_load_shot<T, NDIM, CP>(A, X, g0, lin, so, s0);
-    if (g0 + 1 < g1) adj_load_shot<T, NDIM, CP>(A, X, g0 + 1, lin, so, s1);
+    AdjShot<T, NDIM> s0, s1, s2;
+    adj_load_shot<T, NDIM>(A, g0, off, so, s0);
+    if (g0 + 1 < g1) adj_load_shot<T, NDIM>(A, g0 + 1, off, so, s1);
     for (int g = g0; g < g1; g += 3) {
-        adj_pipe<T, NDIM, CP>(A, X, g, g1, lin, so, fc, fm, fp, s0, s2, gsum);
-        adj_pipe<T, NDIM, CP>(A, X, g + 1, g1, lin, so, fc, fm, fp, s1, s0, gsum);
-        adj_pipe<T, NDIM, CP>(A, X, g + 2, g1, lin, so, fc, fm, fp, s2, s1, gsum);
+        adj_pipe<T, NDIM>(A, g, g1, off, so, fc, fm, fp, s0, s2, gsum);
+        adj_pipe<T, NDIM>(A, g + 1, g1, off, so, fc, fm, fp, s1, s0, gsum);
+        adj_pipe<T, NDIM>(A, g + 2, g1, off, so, fc, fm, fp, s2, s1, gsum);
     }
-    T* gr = A.grad + (int64_t)grp * A.field_stride;
-    gr[lin] += gsum;
+    *adj_ptr(A.grad + (int64_t)N.grp * A.field_stride, off) += gsum;
+}
+
+// The same of the other block classes, whose tiles hold CPML nodes of the axes
+// in the class's bits.  Shots one after the other, each axis's loads clamped
+// instead of branched on: latency hides behind waves.  Three shots' loads in
+// registers, as in the plain blocks, took 256 VGPRs in FP64 3D (one wave per
+// SIMD) and 125 in FP32 2D: 81x73x69 FP64, 2 shots, 126 us per step, 45 so;
+// 554x554 FP32, 32 shots, 38 us, 30 so.  The next shot's fields loaded early, or
+// the accumulator, spill and lose it again.
+template <typename T, int NDIM, typename Off>
+__device__ __forceinline__ void adj_slab_block(const AdjointArgs<T>& A, int lb) {
+    AdjNode N;
+    if (!adj_node<T, NDIM, true>(A, lb, N)) return;
+    const int64_t so[3] = {1, A.px, A.px * A.n[1]};
+    const int64_t i = N.i, j = N.j, k = N.k, h = A.halo;
+    const Off off = (Off)((i + A.px * j + so[2] * k) * (int64_t)sizeof(T));
+    const Off offx = (Off)(i * (int64_t)sizeof(T));
+    const T* f = A.fact;
+    const T fc = adj_at(f, off);
+    T fm[NDIM], fp[NDIM];
+#pragma unroll
+    for (int a = 0; a < NDIM; ++a) {
+        fm[a] = adj_at(f - so[a], off);
+        fp[a] = adj_at(f + so[a], off);
+    }
+    // x: the side and layers differ from lane to lane, and its slabs hold the
+    // layers of row (j, k) together.  y, z: one side and layer per wave, kept
+    // as rows of nodes.
+    AdjCoef<T> C[NDIM];
+    AdjLayers L[NDIM];
+    bool on[NDIM];
+#pragma unroll
+    for (int a = 0; a < NDIM; ++a) {
+        on[a] = (N.cls >> a) & 1;
+        if (!on[a]) continue;
+        C[a] = adj_coef<T>(A, a, a == 0 ? i : (a == 1 ? j : k), L[a]);
+        if (a) on[a] = C[a].ext;
+    }
+    auto row = [&](int a, int layers, int layer) -> int64_t {
+        return a == 1 ? A.px * (layer + layers * k) : A.px * (j + A.n[1] * layer);
+    };
+    // x: fn(side, its slab row's offsets) for the lanes in a CPML range.  2D:
+    // once per side that lanes of the wave lie in, from scalar bases; 3D: with
+    // each lane's own (the scalar form spills: 81x73x69 FP64, 2 shots, 50 and
+    // 56 us per step; 554x554 FP32, 32 shots, 34 and 30 us)
+    const int64_t rx = j + A.n[1] * k;
+    const bool extx = on[0] && C[0].ext, hix = extx && C[0].side;
+    const bool anyhi = __any(hix), anylo = __any(extx && !hix);
+    auto x_sides = [&](int g, auto fn) {
+        const int64_t bx = g * A.xi_stride[0] + h * rx, ax = g * A.psi_stride[0] + (h + 1) * rx;
+        const AdjSide<T>& D0 = A.side[0][0];
+        const AdjSide<T>& D1 = A.side[0][1];
+        if constexpr (NDIM == 2) {
+            if (anylo && extx && !hix) fn(D0.be_rd + bx, D0.be_wr + bx, D0.al_rd + ax, D0.al_wr + ax);
+            if (anyhi && hix) fn(D1.be_rd + bx, D1.be_wr + bx, D1.al_rd + ax, D1.al_wr + ax);
+        } else if (extx) {
+            fn((hix ? D1.be_rd : D0.be_rd) + bx, (hix ? D1.be_wr : D0.be_wr) + bx,
+               (hix ? D1.al_rd : D0.al_rd) + ax, (hix ? D1.al_wr : D0.al_wr) + ax);
+        }
+    };
+    const unsigned es = sizeof(T);
+    T gsum = T(0);
+    for (int g = N.g0; g < N.g1; ++g) {
+        const int64_t fs = (int64_t)g * A.field_stride;
+        AdjVals<T> V[NDIM];
+        AdjShot<T, NDIM> S;
+        adj_load_shot<T, NDIM>(A, g, off, so, S);
+        x_sides(g, [&](const T* be, T*, const T* al, T*) {
+            V[0].b0 = adj_at(be, es * L[0].b0);
+            V[0].b1 = adj_at(be, es * L[0].b1);
+            V[0].b2 = adj_at(be, es * L[0].b2);
+            V[0].alo = adj_at(al, es * L[0].lo);
+            V[0].ahi = adj_at(al, es * L[0].hi);
+        });
+#pragma unroll
+        for (int a = 1; a < NDIM; ++a) {
+            if (!on[a]) continue;
+            const T* be = (C[a].side ? A.side[a][1].be_rd : A.side[a][0].be_rd) + g * A.xi_stride[a];
+            const T* al = (C[a].side ? A.side[a][1].al_rd : A.side[a][0].al_rd) + g * A.psi_stride[a];
+            V[a].b0 = adj_at(be + row(a, (int)h, L[a].b0), offx);
+            V[a].b1 = adj_at(be + row(a, (int)h, L[a].b1), offx);
+            V[a].b2 = adj_at(be + row(a, (int)h, L[a].b2), offx);
+            V[a].alo = adj_at(al + row(a, (int)h + 1, L[a].lo), offx);
+            V[a].ahi = adj_at(al + row(a, (int)h + 1, L[a].hi), offx);
+        }
+        T uc, um[NDIM], up[NDIM];
+        T acc = adj_plain<T, NDIM>(A, fc, fm, fp, S, uc, um, up);
+        x_sides(g, [&](const T*, T*, const T*, T* al) {
+            adj_term(C[0], V[0], um[0], uc, up[0], A.inv_d[0], A.inv_d2[0], adj_ptr(al, es * L[0].lo),
+                     adj_ptr(al, es * L[0].hi), acc);
+        });
+#pragma unroll
+        for (int a = 1; a < NDIM; ++a) {
+            if (!on[a]) continue;
+            T* al = (C[a].side ? A.side[a][1].al_wr : A.side[a][0].al_wr) + g * A.psi_stride[a];
+            adj_term(C[a], V[a], um[a], uc, up[a], A.inv_d[a], A.inv_d2[a],
+                     adj_ptr(al + row(a, (int)h + 1, L[a].lo), offx),
+                     adj_ptr(al + row(a, (int)h + 1, L[a].hi), offx), acc);
+        }
+        *adj_ptr(A.lam0 + fs, off) = acc;
+        // beta^s = bK beta^{s+1} + f lam^s on every slab holding the node
+        x_sides(g, [&](const T*, T* be, const T*, T*) {
+            if (C[0].v1) *adj_ptr(be, es * L[0].b1) = C[0].bK1 * V[0].b1 + fc * acc;
+        });
+#pragma unroll
+        for (int a = 1; a < NDIM; ++a) {
+            if (!on[a] || !C[a].v1) continue;
+            T* be = (C[a].side ? A.side[a][1].be_wr : A.side[a][0].be_wr) + g * A.xi_stride[a];
+            *adj_ptr(be + row(a, (int)h, L[a].b1), offx) = C[a].bK1 * V[a].b1 + fc * acc;
+        }
+        gsum += acc * S.q;
+    }
+    *adj_ptr(A.grad + (int64_t)N.grp * A.field_stride, off) += gsum;
+}
+
+// One reverse step: of the blocks without CPML nodes (KIND 0), with (1), or both
+// (2).  2D takes both in one launch: those with CPML nodes wait on their loads
+// and keep the VALU busy, the others run at the memory's rate, and the two kinds
+// take turns in proportion to their numbers, in groups of one block per XCD
+// (554x554 FP32, 32 shots: 56 us per step in two launches, 52 in one).  In 3D the
+// plain blocks lose more from the other kind's registers (110x100x98 FP64, 4
+// shots, 60 steps' gradient: 21.5 and 23.6 ms).
+template <typename T, int NDIM, typename Off, int KIND>
+__global__ __launch_bounds__(256, (KIND == 0 ? 1 : (sizeof(T) == 8 ? 3 : (NDIM == 2 ? 5 : 4))))
+void adjoint_step(const AdjointArgs<T> A) {
+    const int xcd = (int)blockIdx.x % kNumXcd, q = (int)blockIdx.x / kNumXcd;
+    const int all = (int)gridDim.x / kNumXcd;
+    if constexpr (KIND == 0) {
+        adj_plain_block<T, NDIM, Off>(A, xcd * all + q);
+    } else if constexpr (KIND == 1) {
+        adj_slab_block<T, NDIM, Off>(A, xcd * all + q);
+    } else {
+        const int slab = (A.blocks[1] + kNumXcd - 1) / kNumXcd;
+        const int before = (int)((int64_t)q * slab / all);
+        if ((int)((int64_t)(q + 1) * slab / all) > before)
+            adj_slab_block<T, NDIM, Off>(A, xcd * slab + before);
+        else
+            adj_plain_block<T, NDIM, Off>(A, xcd * (all - slab) + (q - before));
+    }
 }
 
 // Trace cotangent injection of step it0 (0-based) after adjoint_step:

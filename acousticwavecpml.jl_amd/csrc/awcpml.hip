@@ -2669,11 +2669,9 @@ struct AdjBuffers {
     }
 };
 
-// cp = false: the launch over block class 0 (no CPML nodes); true: over
-// classes 1..7.
 template <typename T>
 awcpml::AdjointArgs<T> make_adj_args(const awcpml_plan* P, const AdjBuffers& Bf, const AdjShape& S,
-                                     int lr, int par, const void* q, bool cp) {
+                                     int lr, int par, const void* q) {
     awcpml::AdjointArgs<T> A;
     memset(&A, 0, sizeof A);
     for (int a = 0; a < 3; ++a) A.n[a] = P->n[a];
@@ -2707,7 +2705,8 @@ awcpml::AdjointArgs<T> make_adj_args(const awcpml_plan* P, const AdjBuffers& Bf,
     }
     A.ndim = P->ndim;
     A.nshots = P->nshots;
-    A.group = cp ? S.group_cp : S.group;
+    A.group[0] = S.group;
+    A.group[1] = S.group_cp;
     A.tiles_x = S.tiles_x;
     A.tiles_y = S.tiles_y;
     for (int a = 0; a < 3; ++a) {
@@ -2715,15 +2714,22 @@ awcpml::AdjointArgs<T> make_adj_args(const awcpml_plan* P, const AdjBuffers& Bf,
         A.int_lo[a] = S.int_lo[a];
         A.int_hi[a] = S.int_hi[a];
     }
-    int64_t total = 0;
-    A.cls_start[0] = 0;
-    for (int c = 0; c < 8; ++c) {
-        if (cp == (c > 0)) total += S.class_blocks[c];
-        A.cls_start[c + 1] = cp ? (int)total : 0;
+    A.blocks[0] = (int)S.class_blocks[0];
+    for (int c = 1; c < 8; ++c) {
+        A.cls_start[c] = A.blocks[1];
+        A.blocks[1] += (int)S.class_blocks[c];
     }
-    A.logical_blocks = (int)total;
-    A.grid_blocks = (int)round_up(A.logical_blocks, awcpml::kNumXcd);
     return A;
+}
+
+template <typename T, int NDIM, typename Off, int KIND>
+void launch_adjoint(const awcpml::AdjointArgs<T>& A, hipStream_t stream) {
+    int64_t grid = 0;
+    for (int cp = 0; cp < 2; ++cp)
+        if (KIND == 2 || KIND == cp) grid += round_up(A.blocks[cp], awcpml::kNumXcd);
+    if (grid == 0) return;
+    awcpml::adjoint_step<T, NDIM, Off, KIND>
+        <<<dim3((unsigned)grid), dim3(awcpml::kTileX, kAdjBlockY), 0, stream>>>(A);
 }
 
 template <typename T>
@@ -2866,6 +2872,7 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     io.ndim = P->ndim;
     io.rq = (T*)Bf.rq;
 
+    const bool wide = (uint64_t)P->field_elems * sizeof(T) >= (1ull << 32);  // byte offsets past 32 bits
     int lr = 0, par = 0;
     for (int64_t seg = P->ck_count - 1; seg >= 0; --seg) {
         const int64_t c0 = seg * K, c1 = std::min<int64_t>(c0 + K, nt);
@@ -2875,20 +2882,18 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         P->it = c1;
         for (int64_t s = c1; s > c0; --s) {
             const void* q = (const char*)Bf.q + (size_t)(s - c0 - 1) * fb;
-            awcpml::AdjointArgs<T> A;
-            for (int cp = 0; cp < 2; ++cp) {  // blocks without, then with CPML nodes
-                A = make_adj_args<T>(P, Bf, shape, lr, par, q, cp != 0);
-                if (A.logical_blocks == 0) continue;
-                const dim3 grid(A.grid_blocks), block(awcpml::kTileX, kAdjBlockY);
-                if (P->ndim == 3) {
-                    if (cp) awcpml::adjoint_step<T, 3, true><<<grid, block, 0, P->stream>>>(A);
-                    else awcpml::adjoint_step<T, 3, false><<<grid, block, 0, P->stream>>>(A);
-                } else {
-                    if (cp) awcpml::adjoint_step<T, 2, true><<<grid, block, 0, P->stream>>>(A);
-                    else awcpml::adjoint_step<T, 2, false><<<grid, block, 0, P->stream>>>(A);
-                }
-                HIP_TRY(hipGetLastError());
+            const awcpml::AdjointArgs<T> A = make_adj_args<T>(P, Bf, shape, lr, par, q);
+            if (P->ndim == 2 && wide) launch_adjoint<T, 2, int64_t, 2>(A, P->stream);
+            if (P->ndim == 2 && !wide) launch_adjoint<T, 2, uint32_t, 2>(A, P->stream);
+            if (P->ndim == 3 && wide) {
+                launch_adjoint<T, 3, int64_t, 0>(A, P->stream);
+                launch_adjoint<T, 3, int64_t, 1>(A, P->stream);
             }
+            if (P->ndim == 3 && !wide) {
+                launch_adjoint<T, 3, uint32_t, 0>(A, P->stream);
+                launch_adjoint<T, 3, uint32_t, 1>(A, P->stream);
+            }
+            HIP_TRY(hipGetLastError());
             if (!node_lin.empty()) {
                 io.lam0 = A.lam0;
                 io.q = (const T*)q;
