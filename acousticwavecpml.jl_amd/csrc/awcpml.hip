@@ -179,10 +179,9 @@ struct awcpml_plan {
     int device = 0;
 
     // adjoint: forward-state checkpoints every ck_every steps (state after
-    // c*ck_every steps: the three field buffers, psi of the current parity,
-    // xi), valid until the model, CPML or sources/receivers change
+    // c*ck_every steps, see CkLayout), valid until the model, CPML or
+    // sources/receivers change
     void* ck = nullptr;
-    size_t ck_bytes = 0;  // per checkpoint
     int64_t ck_every = 0, ck_count = 0;
     size_t ck_alloc = 0;
     bool ck_valid = false;
@@ -1225,17 +1224,17 @@ constexpr size_t kAskFreeBytes = 64ull << 20;
 
 // A plan left to the library's choice gets its spare buffers with its first
 // run of several steps; where they do not fit, or would take more than an
-// eighth of the device memory that is free (which the caller may count on), it
-// keeps single steps.
-int auto_spares(awcpml_plan* P, int64_t n) {
+// eighth of the device memory that is free (which the caller may count on; not
+// counting `later` bytes the library is about to need), it keeps single steps.
+int auto_spares(awcpml_plan* P, int64_t n, size_t later = 0) {
     if (!P->tb_auto || n < 2 || P->p_spare || P->spare_failed || !multi_possible(P)) return AWCPML_OK;
     int64_t elems = P->field_elems;
     for (int a = 0; a < P->ndim; ++a) elems += 2 * (P->psi_elems[a] + P->xi_elems[a]);
     const size_t bytes = (size_t)elems * P->nshots * P->esize;
     size_t avail = 0, total = 0;
-    if (bytes > kAskFreeBytes) {
+    if (bytes + later > kAskFreeBytes) {
         HIP_TRY(hipMemGetInfo(&avail, &total));
-        if (bytes > avail / 8) {
+        if (bytes > (avail - std::min(avail, later)) / 8) {
             P->spare_failed = true;
             return AWCPML_OK;
         }
@@ -2584,53 +2583,65 @@ AdjShape adj_shape(const awcpml_plan* P) {
     return S;
 }
 
+// A checkpoint: pold and pcur (and the third field, which the next step only
+// overwrites, where that shows: with sources on Dirichlet nodes, whose values it
+// keeps there, and with segments too short to overwrite it), then the current
+// psi and xi; each piece 256-byte aligned.
 struct CkLayout {
+    int fields;
     size_t field;            // bytes of one field buffer (all shots)
     size_t psi[3], xi[3];    // bytes of one side's slab (all shots)
     size_t total;
 };
 
-CkLayout ck_layout(const awcpml_plan* P) {
+CkLayout ck_layout(const awcpml_plan* P, int64_t every) {
     CkLayout L{};
+    auto room = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    L.fields = every >= 3 && !P->src_on_boundary ? 2 : 3;
     L.field = (size_t)P->field_elems * P->nshots * P->esize;
-    L.total = 3 * L.field;
+    L.total = L.fields * room(L.field);
     for (int a = 0; a < P->ndim; ++a) {
         L.psi[a] = (size_t)P->psi_elems[a] * P->nshots * P->esize;
         L.xi[a] = (size_t)P->xi_elems[a] * P->nshots * P->esize;
-        L.total += 2 * (L.psi[a] + L.xi[a]);
+        L.total += 2 * (room(L.psi[a]) + room(L.xi[a]));
     }
     return L;
 }
 
 // copy the plan state to (save) or from (restore) checkpoint c
 int ck_copy(awcpml_plan* P, int64_t c, bool save) {
-    const CkLayout L = ck_layout(P);
+    const CkLayout L = ck_layout(P, P->ck_every);
     char* base = (char*)P->ck + (size_t)c * L.total;
-    auto mv = [&](void* state, size_t bytes) -> int {
-        if (bytes == 0) return AWCPML_OK;
-        void* dst = save ? (void*)base : state;
-        const void* src = save ? (const void*)state : (const void*)base;
-        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, P->stream));
-        base += bytes;
-        return AWCPML_OK;
-    };
-    int st;
-    const int par = save ? P->par : P->ck_par[c];
-    for (int b = 0; b < 3; ++b)
-        if ((st = mv(P->p[b], L.field))) return st;
-    for (int a = 0; a < P->ndim; ++a)
-        for (int s = 0; s < 2; ++s) {
-            if ((st = mv(P->psi[a][s][par], L.psi[a]))) return st;
-            if ((st = mv(P->xi[a][s], L.xi[a]))) return st;
+    awcpml::CopyPieces K;
+    K.count = 0;
+    uint64_t most = 0;
+    auto mv = [&](void* state, size_t bytes) {
+        if (bytes) {
+            K.src[K.count] = save ? state : base;
+            K.dst[K.count] = save ? base : state;
+            K.bytes[K.count++] = bytes;
         }
-    if (save) {
-        P->ck_rot[c] = P->rot;
-        P->ck_par[c] = P->par;
-    } else {
+        base += (bytes + 255) / 256 * 256;
+        most = std::max<uint64_t>(most, bytes);
+    };
+    if (!save) {
         P->rot = P->ck_rot[c];
         P->par = P->ck_par[c];
         P->it = c * P->ck_every;
     }
+    for (int b = 0; b < L.fields; ++b) mv(P->p[(P->rot + b) % 3], L.field);
+    for (int a = 0; a < P->ndim; ++a)
+        for (int s = 0; s < 2; ++s) {
+            mv(P->psi[a][s][P->par], L.psi[a]);
+            mv(P->xi[a][s], L.xi[a]);
+        }
+    if (save) {
+        P->ck_rot[c] = P->rot;
+        P->ck_par[c] = P->par;
+    }
+    const unsigned blocks = (unsigned)std::min<uint64_t>(4096, most / 4096 + 1);
+    awcpml::copy_pieces<<<dim3(blocks), dim3(256), 0, P->stream>>>(K);
+    HIP_TRY(hipGetLastError());
     return AWCPML_OK;
 }
 
@@ -2937,7 +2948,7 @@ int awcpml_checkpoint_run(awcpml_plan* P, int64_t every) {
     if (every <= 0) every = std::max<int64_t>(1, (int64_t)llround(sqrt((double)P->nt)));
     every = std::min<int64_t>(every, P->nt);
     const int64_t count = (P->nt + every - 1) / every;
-    const CkLayout L = ck_layout(P);
+    const CkLayout L = ck_layout(P, every);
     const size_t need = L.total * (size_t)count;
     if (need > P->ck_alloc) {
         dfree(P->ck);
@@ -2945,12 +2956,17 @@ int awcpml_checkpoint_run(awcpml_plan* P, int64_t every) {
         if ((st = dalloc(&P->ck, need))) return st;
         P->ck_alloc = need;
     }
-    P->ck_bytes = L.total;
     P->ck_every = every;
     P->ck_count = count;
     P->ck_rot.assign(count, 0);
     P->ck_par.assign(count, 0);
     P->ck_valid = false;
+    // what the gradient will allocate beside its checkpoints
+    const AdjShape shape = adj_shape(P);
+    const size_t later = L.field * (size_t)(every + 3) + 2 * (L.total - L.fields * L.field) +
+                         (size_t)P->field_elems * (shape.ngroups_cp * P->esize + 8) +
+                         (size_t)P->n_rec_total * P->nt * P->esize;
+    if ((st = auto_spares(P, every, later))) return st;
     if ((st = awcpml_reset(P))) return st;
     for (int64_t c = 0; c < count; ++c) {
         if ((st = ck_copy(P, c, true))) return st;

@@ -48,4 +48,27 @@ __global__ __launch_bounds__(256) void gather_fact_edge(const T* fact, T* edge, 
     }
 }
 
+// Several buffers copied in one launch: a checkpoint of the forward run is up to
+// 15 of them.  Small ones cost their launch (4.6 us each with hipMemcpyAsync;
+// 81x73x69 FP64, 2 shots: 69 us per checkpoint, 14 so), large ones run at HBM rate
+// either way.  Buffers are 16-byte aligned; sizes are multiples of 4 bytes.
+constexpr int kMaxPieces = 15;
+struct CopyPieces {
+    const void* src[kMaxPieces];
+    void* dst[kMaxPieces];
+    uint64_t bytes[kMaxPieces];
+    int count;
+};
+
+static __global__ __launch_bounds__(256) void copy_pieces(const CopyPieces P) {
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (int q = 0; q < P.count; ++q) {
+        const uint64_t n16 = P.bytes[q] / 16, n4 = P.bytes[q] / 4;
+        for (uint64_t u = first; u < n16; u += stride) ((uint4*)P.dst[q])[u] = ((const uint4*)P.src[q])[u];
+        for (uint64_t u = n16 * 4 + first; u < n4; u += stride)
+            ((uint32_t*)P.dst[q])[u] = ((const uint32_t*)P.src[q])[u];
+    }
+}
+
 }  // namespace awcpml

@@ -49,3 +49,30 @@ def test_reverse_step_tiles(name):
             P.set_adjoint_group(group)
             assert rel_l2(fwi.misfit_gradient(P, [obs] * 5, every=9)[1], 5 * g) <= tol, group
         P.close()
+
+
+@pytest.mark.parametrize("dirichlet", [False, True])
+@pytest.mark.parametrize("nd", [2, 3])
+def test_checkpoints_of_two_and_three_fields(nd, dirichlet):
+    """Segments of 1 and 2 steps and sources on Dirichlet nodes keep the third
+    field; the oracle's gradient either way (FP64, 1e-10 as above), and from
+    every spacing the same forward state afterwards as from single steps."""
+    print("[gpu] checkpoints %dD dirichlet %s" % (nd, dirichlet), flush=True)
+    n = (43, 37) if nd == 2 else (23, 21, 19)
+    case = (small2d if nd == 2 else small3d)(n=n, halo=5, freetop=True, nt=30)
+    case["srcpos"], case["t0s"] = case["srcpos"][:1].copy(), case["t0s"][:1]
+    case["srcpos"][0] = [10.0 * (v // 2) for v in n]
+    if dirichlet:
+        case["srcpos"][0][-1] = 0.0
+    o = oracle_for(case)
+    o.run()
+    obs = 0.5 * o.traces()
+    _, g = o.fwi_gradient(obs)
+    P, Q = plan_from_oracle(o), plan_from_oracle(o)
+    Q.set_time_block(1)
+    for every in (1, 2, 3, 4, 17, 30):
+        for R in (P, Q):
+            assert rel_l2(fwi.misfit_gradient(R, obs, every=every)[1], g) <= 1e-10, every
+        assert np.array_equal(P.field(0, 1), Q.field(0, 1))
+    P.close()
+    Q.close()
