@@ -66,7 +66,9 @@ struct TileArgs {
     int64_t it0;              // 0-based index of the first step
     int steps;
     int io;                   // 0: no sources, no receivers (timing)
-    int tiles_x, tiles_y;
+    // tile (tx, ty) owns the kTileOwnX columns from tx*kTileOwnX - shift_x on and
+    // the OY rows from 1 + ty*OY - shift_y on, as far as they are interior
+    int tiles_x, tiles_y, shift_x, shift_y;
     // tiles [ix0, ix1) x [iy0, iy1) lie wholly inside the domain and outside
     // the CPML slabs; a launch takes those (CP = false), the others, or all
     // (the range is then empty)
@@ -165,8 +167,9 @@ __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ?
     const int lane = (int)threadIdx.x;
     const int wy = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int nx = (int)A.nx, ny = (int)A.ny, h = (int)A.halo;
-    const int x = tx * kTileOwnX - kTileHalo + lane;
-    const int yt = 1 + ty * OY - kTileHalo;   // first row of the tile
+    const int xt = tx * kTileOwnX - B.shift_x - kTileHalo;   // first column of the tile
+    const int x = xt + lane;
+    const int yt = 1 + ty * OY - B.shift_y - kTileHalo;      // first row of the tile
     const int y0 = yt + wy * R;               // first row of the wave
     const bool inx = x >= 1 && x <= nx - 2;
     const int xc = x < 0 ? 0 : (x > nx - 1 ? nx - 1 : x);
@@ -279,17 +282,18 @@ __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ?
     bool src = false;
     for (int e = s0; e < s1; ++e) {
         const int64_t xy = B.src_xy[e];
-        const int dx = (int)(xy & 0xffffffff) - (tx * kTileOwnX - kTileHalo), dy = (int)(xy >> 32) - yt;
+        const int dx = (int)(xy & 0xffffffff) - xt, dy = (int)(xy >> 32) - yt;
         src = src || (dx >= 0 && dx < kTileX && dy >= 0 && dy < TY);
     }
-    const int oy0 = 1 + ty * OY, oy1 = oy0 + OY < ny - 1 ? oy0 + OY : ny - 1;  // owned rows
+    const int ye = yt + kTileHalo + OY;
+    const int oy0 = yt + kTileHalo > 1 ? yt + kTileHalo : 1, oy1 = ye < ny - 1 ? ye : ny - 1;  // owned rows
     const int q0 = B.rec_band[shot * B.bands + oy0 / kRecBand];
     const int q1 = B.io ? B.rec_band[shot * B.bands + (oy1 - 1) / kRecBand + 1] : q0;
     const int tid = wy * kTileX + lane;
     bool mine = false;
     for (int q = q0 + tid; q < q1; q += 64 * W) {
         const int64_t xy = B.rec_xy[q];
-        const int rx = (int)(xy & 0xffffffff) - tx * kTileOwnX, ry = (int)(xy >> 32);
+        const int rx = (int)(xy & 0xffffffff) - xt - kTileHalo, ry = (int)(xy >> 32);
         mine = mine || (rx >= 0 && rx < kTileOwnX && ry >= oy0 && ry < oy1);
     }
     const bool rec = __syncthreads_or(mine);
@@ -379,7 +383,7 @@ __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ?
             __syncthreads();
             for (int q = q0 + tid; q < q1; q += 64 * W) {
                 const int64_t xy = B.rec_xy[q];
-                const int rx = (int)(xy & 0xffffffff) - tx * kTileOwnX, ry = (int)(xy >> 32);
+                const int rx = (int)(xy & 0xffffffff) - xt - kTileHalo, ry = (int)(xy >> 32);
                 if (rx >= 0 && rx < kTileOwnX && ry >= oy0 && ry < oy1)
                     B.traces[(int64_t)B.rec_idx[q] * B.nt + B.it0 + s] = rows[ry - yt][rx + kTileHalo];
             }

@@ -115,3 +115,33 @@ def test_batch_accepts_plans_that_ran_on_their_own():
             assert np.array_equal(P.traces(), want)
     for P in plans:
         P.close()
+
+
+# tiles that begin before the corner: the same grid size modulo 48 at different
+# halos and idle sides moves the beginning through its whole range
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n,halo,freetop", [((171, 150), 8, False), ((200, 163), 11, True), ((207, 197), 20, False),
+                                            ((175, 191), 3, True), ((193, 162), 15, False)])
+def test_moved_tiles_equal_single_steps(n, halo, freetop, dtype):
+    print("[gpu] moved tiles %s %d %s" % (n, halo, dtype), flush=True)
+    o = _oracle(_case(n, halo, freetop, 21))
+    pts = _points(n)
+    shots = 520
+    srcs = [pts[[(5 * s) % len(pts)]] for s in range(shots)]
+    P = _plan(o, dtype=dtype, nshots=shots, srcs=srcs)
+    for s in range(shots):
+        P.set_receivers(s, pts[s % 3::3])
+    show = range(0, shots, 37)
+
+    def run(k):
+        P.reset()
+        P.advance(k)
+        P.advance(o.nt - k)
+        return [[P.traces(s)] + [P.field(s, f) for f in range(3)] for s in show]
+
+    moved = [run(0), run(11)]
+    P.set_time_block(1)
+    one = run(0)
+    for m in moved:
+        _same(m, one)
+    P.close()
