@@ -760,19 +760,6 @@ bool tile_ok(const awcpml_plan* P) {
 
 int two_rows_default(int ndim, int dtype) { return ndim == 2 ? 4 : (dtype == AWCPML_F64 ? 8 : 16); }
 
-// The chunk length of a plan's share of two-step batch launches (W waves per
-// block), and of 3D plans where it is set.
-int two_march(const awcpml_plan* P, int W) {
-    if (P->tb_march > 0) return P->tb_march;
-    if (P->ndim == 2) return (int)std::max<int64_t>(8, std::min<int64_t>(64, (P->n[1] - 2) / 16));
-    // enough blocks to fill 256 CUs several times over
-    const int64_t tiles = ((P->n[0] - 2 + awcpml::kOwnX - 1) / awcpml::kOwnX) *
-                          ((P->n[1] - 2 + W - 3) / (W - 2)) * P->nshots;
-    const int64_t interior = P->n[2] - 2;
-    const int64_t want = std::max<int64_t>(1, (2048 + tiles - 1) / tiles);
-    return (int)std::max<int64_t>(16, std::min<int64_t>((interior + want - 1) / want, 128));
-}
-
 // March chunks of a two-step launch (chunk_start[0..count]), or 0 for
 // uniform chunks of ml planes.  A chunk reads one plane beyond each end
 // (step t+1 there), so the CPML layers 1..halo of each absorbing side of
@@ -800,83 +787,103 @@ int two_chunk_list(const awcpml_plan* P, int ml, int* starts) {
     return count;
 }
 
-// Waves per block and chunk length of a 3D plan's two-step launches where they
-// are not set: the shape whose slowest XCD is done first.  An XCD works through
-// an eighth of the blocks in order (x, y tiles, then chunks, then shots) on 32
-// CUs; a block's time is its planes (1.3 times in the CPML layers) and 20 (FP32:
-// 16) more for its start and the planes at its ends.  FP64 blocks of 8 waves and
-// FP32 blocks of 16 have a CU to themselves; two FP32 blocks of 8 share one and
-// are 5 % faster for their rows.  Up to 256 blocks are placed one by one, more
-// take their mean and half a block.  FP64 chunks stay below 49 planes: blocks
-// that march further drift apart and find less in L2 (450x430x300: 461 us per
-// step at 40 planes, 534 at 96; 298^3, 3 shots: 627 and 718), unless whole shots
-// or halves of them share out evenly among the XCDs (298^3, 4 shots: 816 and
-// 785; 200x180x190, 8 shots: 560 and 539).
+// Chunk length, and waves per block where rows = 0, of the two-step launches of
+// a 3D plan, or of several in a batch, where they are not set: the shape whose
+// slowest XCD is done first.  An XCD works through an eighth of the blocks in
+// order (x, y tiles, then chunks, shots, plans) on 32 CUs; a block's time is its
+// planes (1.3 times in the CPML layers) and 20 (FP32: 16) more for its start and
+// the planes at its ends.  FP64 blocks of 8 waves and FP32 blocks of 16 have a CU
+// to themselves; two FP32 blocks of 8 share one and are 5 % faster for their
+// rows.  Up to 256 blocks are placed one by one, more take their mean and half a
+// block.  FP64 chunks stay below 49 planes: blocks that march further drift apart
+// and find less in L2 (450x430x300: 461 us per step at 40 planes, 534 at 96;
+// 298^3, 3 shots: 627 and 718), unless whole shots or halves of them share out
+// evenly among the XCDs (298^3, 4 shots: 816 and 785; 200x180x190, 8 shots: 560
+// and 539).
 // On 39 grids and shot counts from 30x32x28 to 450x430x300 nodes, every shape
-// timed, this is 1.4 % above the best shape on average and 19 % at worst; 2048
-// blocks of 16 to 128 planes, the rule of batches, are up to 40 % above it.
-void two_shape(const awcpml_plan* P, int* rows, int* march) {
-    const bool f64 = P->dtype == AWCPML_F64;
-    const bool slabs = P->halo > 0 && (P->active[2][0] || P->active[2][1]);
+// timed, this is 1.4 % above the best shape on average and 19 % at worst; a fixed
+// target of 2048 blocks of 16 to 128 planes is up to 40 % above it (a batch of
+// 170^3, 234^3 and 298^3: FP32 233 and 216 us per step, FP64 497 and 445).
+void two_shape(const std::vector<const awcpml_plan*>& plans, int rows, int* rows_out, int* march) {
+    const bool f64 = plans[0]->dtype == AWCPML_F64;
+    const bool even = plans.size() == 1 && plans[0]->nshots % 4 == 0;
+    std::vector<std::pair<int64_t, double>> runs;  // blocks of one chunk: how many, and the time of one
+    std::vector<double> busy;
     double best = 0;
     for (int W : {16, 8, 4}) {
-        if (P->tb_rows > 0 ? W != P->tb_rows : (W == 4 || (f64 && W == 16))) continue;
-        const int64_t tiles = ((P->n[0] - 2 + awcpml::kOwnX - 1) / awcpml::kOwnX) *
-                              ((P->n[1] - 2 + W - 3) / (W - 2));
+        if (rows > 0 ? W != rows : (W == 4 || (f64 && W == 16))) continue;
         const int share = std::max(1, (f64 ? 8 : 16) / W);  // blocks on a CU together
         const size_t slots = (size_t)32 * share;
         for (int ml : {4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 36, 40, 48, 56, 64, 80, 96}) {
-            if (f64 && ml > 48 && P->nshots % 4 != 0) break;
-            int starts[awcpml::kMaxChunks2 + 1];
-            int64_t n = two_chunk_list(P, ml, starts);
-            const bool uniform = n == 0;
-            if (uniform) n = (P->n[2] - 2 + ml - 1) / ml;
-            auto block_time = [&](int64_t c) {
-                const int64_t z0 = uniform ? 1 + c * ml : starts[c];
-                const int64_t z1 = uniform ? std::min<int64_t>(z0 + ml, P->n[2] - 1) : starts[c + 1];
-                const bool layer = slabs && (uniform || (P->active[2][0] && z1 <= P->halo + 2) ||
-                                             (P->active[2][1] && z0 >= P->n[2] - P->halo - 2));
-                return (f64 ? 20 : 16) + (layer ? 1.3 : 1.0) * (double)(z1 - z0);
-            };
-            const int64_t total = tiles * n * P->nshots;
+            if (f64 && ml > 48 && !even) break;
+            runs.clear();
+            int64_t total = 0;
+            double sum = 0, longest = 0;
+            for (const awcpml_plan* P : plans) {
+                const int len = P->tb_march > 0 ? P->tb_march : ml;
+                const bool slabs = P->halo > 0 && (P->active[2][0] || P->active[2][1]);
+                const int64_t tiles = ((P->n[0] - 2 + awcpml::kOwnX - 1) / awcpml::kOwnX) *
+                                      ((P->n[1] - 2 + W - 3) / (W - 2));
+                int starts[awcpml::kMaxChunks2 + 1];
+                int64_t n = two_chunk_list(P, len, starts);
+                const bool uniform = n == 0;
+                if (uniform) n = (P->n[2] - 2 + len - 1) / len;
+                const size_t first = runs.size();
+                for (int64_t c = 0; c < n; ++c) {
+                    const int64_t z0 = uniform ? 1 + c * len : starts[c];
+                    const int64_t z1 = uniform ? std::min<int64_t>(z0 + len, P->n[2] - 1) : starts[c + 1];
+                    const bool layer = slabs && (uniform || (P->active[2][0] && z1 <= P->halo + 2) ||
+                                                 (P->active[2][1] && z0 >= P->n[2] - P->halo - 2));
+                    const double t = (f64 ? 20 : 16) + (layer ? 1.3 : 1.0) * (double)(z1 - z0);
+                    runs.push_back({tiles, t});
+                    sum += t * (double)(tiles * P->nshots);
+                    longest = std::max(longest, t);
+                }
+                for (int64_t q = n; q < n * P->nshots; ++q) runs.push_back(runs[first + (size_t)(q % n)]);
+                total += tiles * n * P->nshots;
+            }
             const int64_t per = (total + awcpml::kNumXcd - 1) / awcpml::kNumXcd;
             double slowest = 0;
             if (per > 256 * share) {
-                double sum = 0, longest = 0;
-                for (int64_t c = 0; c < n; ++c) {
-                    sum += block_time(c) / (double)n;
-                    longest = std::max(longest, block_time(c));
-                }
-                slowest = sum * (double)per / (double)slots + longest / 2;
+                slowest = sum / (double)total * (double)per / (double)slots + longest / 2;
             } else {
-                for (int64_t x0 = 0; x0 < total; x0 += per) {
-                    std::vector<double> busy(slots, 0.0);  // a heap, first free on top
-                    for (int64_t q = x0; q < std::min(total, x0 + per); ++q) {
+                int64_t done = 0;  // blocks placed
+                for (const auto& run : runs)
+                    for (int64_t q = 0; q < run.first; ++q, ++done) {
+                        if (done % per == 0) busy.assign(slots, 0.0);  // a heap, first free on top
                         std::pop_heap(busy.begin(), busy.end(), std::greater<>());
-                        busy.back() += block_time(q / tiles % n);
+                        busy.back() += run.second;
                         slowest = std::max(slowest, busy.back());
                         std::push_heap(busy.begin(), busy.end(), std::greater<>());
                     }
-                }
             }
             if (!f64 && W == 8) slowest *= 0.95;
             if (best == 0 || slowest < best) {
                 best = slowest;
-                *rows = W;
+                *rows_out = W;
                 *march = ml;
             }
         }
     }
 }
 
+// The chunk length of 2D two-step launches in a batch, and of single plans as
+// they report it.
+int march_2d(const awcpml_plan* P) {
+    if (P->tb_march > 0) return P->tb_march;
+    return (int)std::max<int64_t>(8, std::min<int64_t>(64, (P->n[1] - 2) / 16));
+}
+
 void two_tiling(const awcpml_plan* P, int* rows, int* march, int* prefetch) {
-    if (P->ndim == 3 && P->tb_march == 0) {
-        if (P->two_march == 0) two_shape(P, &P->two_rows, &P->two_march);
+    *rows = P->tb_rows > 0 ? P->tb_rows : two_rows_default(P->ndim, P->dtype);
+    if (P->ndim == 2) {
+        *march = march_2d(P);
+    } else if (P->tb_march > 0) {
+        *march = P->tb_march;
+    } else {
+        if (P->two_march == 0) two_shape({P}, P->tb_rows, &P->two_rows, &P->two_march);
         *rows = P->two_rows;
         *march = P->two_march;
-    } else {
-        *rows = P->tb_rows > 0 ? P->tb_rows : two_rows_default(P->ndim, P->dtype);
-        *march = two_march(P, *rows);
     }
     *prefetch = P->tb_prefetch > 0 ? P->tb_prefetch : 2;
 }
@@ -1416,6 +1423,9 @@ int batch_tables_t(awcpml_batch* B, const Roles& R, RoleTables* out) {
     for (auto* P : B->plans) two = two && P->p_spare;
     int W, pf;
     batch_two_shape(B, &W, &pf);
+    int common = 0;  // chunk length of the plans that set none
+    if (two && B->ndim == 3)
+        two_shape(std::vector<const awcpml_plan*>(B->plans.begin(), B->plans.end()), W, &W, &common);
     std::vector<StencilArgs<T>> args((size_t)6 * np);
     std::vector<awcpml::Stencil2Args<T>> args2(two ? (size_t)6 * np : 0);
     std::vector<awcpml::IoArgs<T>> io((size_t)6 * np);
@@ -1425,7 +1435,7 @@ int batch_tables_t(awcpml_batch* B, const Roles& R, RoleTables* out) {
         set_layout(P, roles_layout(P, R, 0));
         for (int v = 0; v < 6; ++v) args[(size_t)v * np + q] = make_args<T>(P, v % 3, v % 2);
         if (two) {
-            const int ml = two_march(P, W);
+            const int ml = B->ndim == 2 ? march_2d(P) : P->tb_march > 0 ? P->tb_march : common;
             for (int v = 0; v < 6; ++v) {
                 P->rot = v % 3;
                 P->par = v % 2;

@@ -92,3 +92,34 @@ def test_default_graph_gradient_and_limits():
         P.advance(o.nt)
         _same(_state(P, 1), auto)
         P.close()
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_batch_shape_and_plans_that_ran(dtype):
+    """Batches in the shape found for all their plans (one plan sets its own
+    chunk length), and of plans that ran by themselves before."""
+    print("[gpu] default 3D launches: batch %s" % dtype, flush=True)
+    os_ = [_oracle(small3d(n=n, halo=h, freetop=f, nt=21))
+           for n, h, f in (((37, 29, 23), 5, True), ((70, 19, 41), 4, False), ((24, 50, 90), 3, False))]
+    plans = [_plan(o, dtype=dtype, nshots=k) for o, k in zip(os_, (1, 3, 2))]
+    nt = min(o.nt for o in os_)
+    want = []
+    for P in plans:
+        P.advance(nt)
+        want.append([P.traces(s)[:nt] for s in range(P.nshots)])
+
+    def check():
+        with awcpml.Batch(plans) as B:
+            B.reset()
+            B.advance(nt)
+            for P, w in zip(plans, want):
+                assert all(np.array_equal(P.traces(s)[:nt], w[s]) for s in range(P.nshots))
+            return B.time_block()
+
+    assert check()[0] == 1  # nothing asked for two steps; the plans are not at home
+    for P, march in zip(plans, (0, 7, 0)):
+        P.reset()
+        P.set_time_block(2, 0, march)
+    assert check()[:2] == (2, 8 if dtype == "f64" else 16)
+    for P in plans:
+        P.close()
