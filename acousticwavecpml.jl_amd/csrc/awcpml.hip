@@ -1025,7 +1025,7 @@ int launch_tile_t(awcpml_plan* P, int64_t it0, int steps, void* q, bool io = tru
     if (rows == 64) {
         // where the tiles begin: so that as few as possible hold CPML nodes,
         // which cost 2.6 times a plain tile (halo 20, from the corner and so:
-        // 1066x1066 FP32, 64 shots, 129 and 109 of 529 tiles, 611 and 595 us per
+        // 1066x1066 FP32, 64 shots, 129 and 109 of 529 tiles, 610 and 590 us per
         // launch; 2001x1501 FP64, 3 shots, 2.86 for 3.09 ms of 160 steps).  x in
         // steps of 16 columns, whose rows stay as aligned as the corner's (8:
         // 554x554, 32 shots, gradient 48.4 ms, 16: 47.0, corner: 47.9).

@@ -168,7 +168,8 @@ int awcpml_get_shot_group(const awcpml_plan *plan, int *shot_group);
  * exactly as the reference's does).  Results are bit-identical to one step
  * per launch.  steps = 1: one step per launch.  A plan for which this is
  * never called takes launches of several steps where those apply and their
- * spare buffers fit (allocated with the first run of two steps or more).
+ * spare buffers need at most an eighth of the free device memory (allocated
+ * with the first run of two steps or more).
  * 3D launch shape: block_rows is the number of wavefronts per block, 4, 8
  * or 16 (the block updates block_rows-2 rows and recomputes the first step
  * on the two outer ones), march_len the chunk along z, prefetch the planes
