@@ -999,6 +999,11 @@ int launch_tile_t(awcpml_plan* P, int64_t it0, int steps, void* q, bool io = tru
     B.p2 = (T*)P->p_spare;
     B.q = (T*)q;
     B.q_step = P->field_elems * P->nshots;
+    // the reverse steps read a segment's q fields last first: where they exceed
+    // the 256 MiB of the last-level cache, storing them past it leaves it to the
+    // state (554x554 FP32, 32 shots, 790 MB a segment: gradient 46.6 ms, 45.0 so;
+    // 400x380, 16 shots, 117 MB: 9.95, but 10.25 if it did)
+    B.q_stream = (uint64_t)P->ck_every * (uint64_t)B.q_step * sizeof(T) > (256ull << 20);
     const char* lists = (const char*)P->d_io_lists;
     B.src_xy = (const int64_t*)(lists + P->tile_src_xy);
     B.src_wav = (const T*)P->d_src_wav;

@@ -60,8 +60,10 @@ template void launch_plan_stencil2<AWCPML_REAL>(const Stencil2Args<AWCPML_REAL>&
 #else
 template <typename T, int R, int W, int KIND>
 static void go_tile(const TileArgs<T>& B, const LaunchShape& L) {
-    if (B.q) stencil2d_tile<T, R, W, KIND, true><<<L.grid, dim3(kTileX, W), 0, L.stream>>>(B);
-    else stencil2d_tile<T, R, W, KIND, false><<<L.grid, dim3(kTileX, W), 0, L.stream>>>(B);
+    const dim3 block(kTileX, W);
+    if (!B.q) stencil2d_tile<T, R, W, KIND, 0><<<L.grid, block, 0, L.stream>>>(B);
+    else if (!B.q_stream) stencil2d_tile<T, R, W, KIND, 1><<<L.grid, block, 0, L.stream>>>(B);
+    else stencil2d_tile<T, R, W, KIND, 2><<<L.grid, block, 0, L.stream>>>(B);
 }
 
 template <typename T>

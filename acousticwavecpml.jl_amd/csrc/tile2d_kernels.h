@@ -52,6 +52,7 @@ struct TileArgs {
     // elements apart; null = off
     T* q;
     int64_t q_step;
+    int q_stream;             // 1: q is stored past the caches
     const int64_t* src_xy;    // source nodes of all shots (x | y << 32)
     const T* src_wav;         // nt values per source
     const int* src_start;     // nshots+1 CSR offsets
@@ -148,8 +149,8 @@ enum TileKind {
     kTileOverlap,  // any tile and grid: every slab node keeps both its edges
 };
 
-// Q: d(pnew)/d(fact) outputs.
-template <typename T, int R, int W, int KIND, bool Q>
+// Q: d(pnew)/d(fact) outputs (1), past the caches (2).
+template <typename T, int R, int W, int KIND, int Q>
 __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ? 8 : 4) void stencil2d_tile(const TileArgs<T> B) {
     constexpr int TY = R * W, OY = TY - 2 * kTileHalo;
     constexpr bool CP = KIND != kTilePlain, OV = KIND == kTileOverlap;
@@ -359,8 +360,12 @@ __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ?
             p[r] = v;
             if (Q) {
                 const int k = wy * R + r;
-                if (ownx && k >= kTileHalo && k < TY - kTileHalo && (!CP || (imask & (1u << r))))
-                    stg(B.q + fo + s * B.q_step, col + (uint32_t)(y0 + r) * pitch, lap + slab);
+                if (ownx && k >= kTileHalo && k < TY - kTileHalo && (!CP || (imask & (1u << r)))) {
+                    T* q = B.q + fo + s * B.q_step;
+                    const uint32_t off = col + (uint32_t)(y0 + r) * pitch;
+                    if constexpr (Q == 2) stg_stream(q, off, lap + slab);
+                    else stg(q, off, lap + slab);
+                }
             }
         }
         if (src) {
@@ -399,8 +404,16 @@ __global__ __launch_bounds__(64 * W, KIND == kTileOverlap ? 2 : sizeof(T) == 4 ?
         if (k < kTileHalo || k >= TY - kTileHalo || (CP && !(imask & (1u << r)))) continue;
         if (!ownx) continue;
         const uint32_t off = col + (uint32_t)j * pitch;
-        stg(B.p1 + fo, off, o[r]);
-        stg(B.p2 + fo, off, p[r]);
+        if constexpr (KIND == kTilePlain) {
+            // large grids: next read in the following launch, and the tiles'
+            // shared margins stay in L2 (2001x1501 FP64, 3 shots, 160 steps:
+            // 2.87 ms, 2.71 so; 1066x1066 FP32, 64 shots, 400 steps: 33.0, 32.7)
+            stg_stream(B.p1 + fo, off, o[r]);
+            stg_stream(B.p2 + fo, off, p[r]);
+        } else {
+            stg(B.p1 + fo, off, o[r]);
+            stg(B.p2 + fo, off, p[r]);
+        }
         if (CP) {
             if (nodex) {
                 T* pw = (sx ? A.side[0][1].psi_wr : A.side[0][0].psi_wr) + shot * A.psi_stride[0];

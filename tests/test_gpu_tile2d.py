@@ -145,3 +145,19 @@ def test_moved_tiles_equal_single_steps(n, halo, freetop, dtype):
     for m in moved:
         _same(m, one)
     P.close()
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_gradient_of_segments_past_the_cache(dtype):
+    """q fields of one segment above 256 MiB are stored past the caches."""
+    o = _oracle(_case((300, 290), 6, False, 20))
+    o.run()
+    shots = 60
+    P = _plan(o, dtype=dtype, nshots=shots, srcs=[o.positions()[0]] * shots)
+    obs = [0.5 * o.traces()] * shots
+    assert 300 * 290 * shots * o.nt * (8 if dtype == "f64" else 4) > 256 << 20
+    auto = awcpml.fwi.misfit_gradient(P, obs, every=o.nt)
+    P.set_time_block(1)
+    one = awcpml.fwi.misfit_gradient(P, obs, every=o.nt)
+    assert auto[0] == one[0] and np.array_equal(auto[1], one[1])
+    P.close()
