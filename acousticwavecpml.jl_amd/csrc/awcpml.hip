@@ -2528,7 +2528,7 @@ int awcpml_get_tiling(const awcpml_plan* P, int* block_y, int* march_len, int* p
 // Adjoint (FWI gradient): checkpointed forward, then per checkpoint
 // segment a forward replay that stores q^s = d(pnew)/d(fact) for every
 // step of the segment, followed by the reverse-time steps of the segment
-// (adjoint_kernels.h).  Memory: ck_count checkpoints of 3 fields + slabs,
+// (adjoint_kernels.h).  Memory: ck_count checkpoints (CkLayout),
 // ck_every q fields, 3 adjoint fields, 2 x slabs, one gradient per shot
 // group.
 // ---------------------------------------------------------------------
@@ -2931,8 +2931,9 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     for (int64_t seg = P->ck_count - 1; seg >= 0; --seg) {
         const int64_t c0 = seg * K, c1 = std::min<int64_t>(c0 + K, nt);
         if ((st = ck_copy(P, seg, false))) return st;
-        // replay, storing q^s (bit-identical whatever the steps per launch)
-        if ((st = enqueue_steps(P, c0, c1 - c0, false, (char*)Bf.q))) return st;
+        // replay, storing q^s (bit-identical whatever the steps per launch);
+        // the first segment's is the state the plan is left in
+        if ((st = enqueue_steps(P, c0, c1 - c0, seg == 0, (char*)Bf.q))) return st;
         P->it = c1;
         for (int64_t s = c1; s > c0; --s) {
             const void* q = (const char*)Bf.q + (size_t)(s - c0 - 1) * fb;

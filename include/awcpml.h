@@ -275,9 +275,10 @@ int awcpml_batch_time_stencil2(awcpml_batch *batch, int nlaunches, double *ms_to
 /* ------------------------------------------------------------------ */
 
 /* Reset the plan and run all nt steps, keeping a checkpoint of the forward
- * state (the three field buffers, psi, xi) every `every` steps (<= 0:
+ * state (pold, pcur, psi, xi, and pnew where the next steps read it: for
+ * every < 3 or a source on a Dirichlet node) every `every` steps (<= 0:
  * round(sqrt(nt))).  The traces of the run are then available as after
- * awcpml_advance.  Device memory: ceil(nt/every) x (3 fields + slabs).
+ * awcpml_advance.  Device memory: ceil(nt/every) x (2 or 3 fields + slabs).
  * Needs >= 2*halo+4 points on every absorbing axis.  The checkpoints stay
  * valid until the model, the CPML coefficients, the sources or the
  * receivers change.  This is the forward half of a reverse-mode rule: the
@@ -295,7 +296,8 @@ int awcpml_checkpoint_run(awcpml_plan *plan, int64_t every);
  * the forward is replayed (storing d(pnew)/d(fact) for each step) and then
  * stepped back in reverse time.  Receivers on Dirichlet nodes carry no
  * gradient (those nodes do not depend on fact).  Leaves the plan's forward
- * state at an intermediate step; the traces are unchanged. */
+ * state (all three fields) at step `every` of awcpml_checkpoint_run; the
+ * traces are unchanged. */
 int awcpml_adjoint(awcpml_plan *plan, const double *trace_bar, int64_t count, double *fact_bar);
 
 /* ------------------------------------------------------------------ */

@@ -1,0 +1,50 @@
+"""Plans and batches left to the library's choice of launches: what a call left
+behind, accepted, refused or timed with one step per launch it does with several
+(three fields after a gradient, batches whose plans run alone in between, timed
+runs, memory that has run short).
+
+Everything is compared value for value with a plan set to single steps, or with
+the same call made another way.
+"""
+import numpy as np
+import pytest
+
+import awcpml
+from cases import small2d, small3d
+from test_gpu_two_step import _oracle, _plan, _same, _state
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(nd, nt=30, freetop=True, n=None):
+    """One source inside, so that launches of several steps apply."""
+    n = n or ((61, 53) if nd == 2 else (37, 29, 23))
+    case = (small2d if nd == 2 else small3d)(n=n, halo=5, freetop=freetop, nt=nt)
+    case["srcpos"], case["t0s"] = np.array([[10.0 * (v // 2) for v in n]]), case["t0s"][:1]
+    return case
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("nd", [2, 3])
+def test_state_after_gradient(nd, dtype):
+    """All three fields and the step count after a gradient, and the run that
+    goes on from there."""
+    print("[gpu] state after a gradient %dD %s" % (nd, dtype), flush=True)
+    o = _oracle(_case(nd))
+    o.run()
+    obs = [0.5 * o.traces()] * 2
+    plans = [_plan(o, dtype=dtype, nshots=2, srcs=[o.positions()[0]] * 2) for _ in range(2)]
+    plans[1].set_time_block(1)
+    for every in (1, 2, 3, 4, 5, 9, 11, 17, 30):
+        got = []
+        for P in plans:
+            awcpml.fwi.misfit_gradient(P, obs, every=every)
+            left = _state(P, 2)
+            at = P.steps_done()
+            P.advance(min(4, o.nt - at))
+            got.append((at, left, _state(P, 2)))
+        assert got[0][0] == got[1][0] == every
+        _same(got[0][1], got[1][1])
+        _same(got[0][2], got[1][2])
+    for P in plans:
+        P.close()
