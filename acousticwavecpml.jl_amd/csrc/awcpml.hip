@@ -1222,7 +1222,9 @@ int plan_graph(awcpml_plan* P, int64_t n, GraphEntry** out) {
 
 // The spare buffers of multi-step launches (one field, one psi and one xi per
 // CPML side).  They start as zeros, like every buffer after a reset, and are
-// allocated before any such launch, so the layout is still home.
+// allocated before any such launch, so the layout is still home.  Batches that
+// hold the plan stay valid: their single steps do not touch the spares, and
+// two-step batches have their plans' spares from awcpml_set_time_block.
 int alloc_spares(awcpml_plan* P) {
     if (P->p_spare) return AWCPML_OK;
     void* f = nullptr;
@@ -1256,7 +1258,6 @@ int alloc_spares(awcpml_plan* P) {
             P->home.psi[a][s][2] = P->psi_spare[a][s] = psi[a][s];
             P->home.xi[a][s][1] = P->xi_spare[a][s] = xi[a][s];
         }
-    ++P->gen;
     return AWCPML_OK;
 }
 

@@ -11,7 +11,7 @@ import pytest
 
 import awcpml
 from cases import small2d, small3d
-from test_gpu_two_step import _oracle, _plan, _same, _state
+from test_gpu_two_step import _batch_state, _oracle, _plan, _same, _state
 
 pytestmark = pytest.mark.gpu
 
@@ -47,4 +47,33 @@ def test_state_after_gradient(nd, dtype):
         _same(got[0][1], got[1][1])
         _same(got[0][2], got[1][2])
     for P in plans:
+        P.close()
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("own", ["advance", "checkpoint"])
+def test_batch_goes_on_after_a_plan_ran_on_its_own(nd, own):
+    """A plan's first run of its own, and its reset, leave a batch that holds it
+    as it was."""
+    print("[gpu] batch after a plan's own run %dD %s" % (nd, own), flush=True)
+    os_ = [_oracle(_case(nd, nt)) for nt in (30, 26)]
+    ref = [_plan(o) for o in os_]
+    for P, o in zip(ref, os_):
+        P.set_time_block(1)
+        P.advance(o.nt)
+    plans = [_plan(o) for o in os_]
+    with awcpml.Batch(plans) as B:
+        plans[0].reset()
+        plans[0].advance(12) if own == "advance" else plans[0].checkpoint_run(6)
+        plans[0].reset()
+        B.advance(30)
+        _same(_batch_state(plans), _batch_state(ref))
+        B.set_graph(True)
+        for _ in range(2):
+            B.run()
+            _same(_batch_state(plans), _batch_state(ref))
+        B.set_time_block(2)
+        B.run()
+        _same(_batch_state(plans), _batch_state(ref))
+    for P in plans + ref:
         P.close()
