@@ -156,6 +156,7 @@ struct awcpml_plan {
     size_t tile_src_xy = 0, tile_rec_xy = 0, tile_rec_idx = 0, tile_rec_band = 0;
 
     int64_t it = 0;   // steps done
+    int uncounted = 0;   // buffer rotations since the reset that are not in it
     int rot = 0;      // p[rot] = pold, p[rot+1] = pcur, p[rot+2] = pnew
     int par = 0;      // psi[..][par] = previous step
 
@@ -1706,11 +1707,65 @@ int batch_prepare(awcpml_batch* B, int64_t it0, int64_t n) {
     return AWCPML_OK;
 }
 
+// Move the plan's state into the buffers of layout L (the same buffers in other
+// roles): every field, the current psi, and xi; what the next step overwrites
+// stays where it is.
+int settle(awcpml_plan* P, const BufLayout& L) {
+    const BufLayout C = get_layout(P);
+    if (C == L) return AWCPML_OK;
+    struct Move {
+        void *from, *to;
+        size_t bytes;
+    };
+    std::vector<Move> todo;
+    auto add = [&](void* from, void* to, size_t bytes) {
+        if (from != to && bytes) todo.push_back({from, to, bytes});
+    };
+    for (int b = 0; b < 3; ++b)
+        add(C.p[(C.rot + b) % 3], L.p[(L.rot + b) % 3], (size_t)P->field_elems * P->nshots * P->esize);
+    for (int a = 0; a < P->ndim; ++a)
+        for (int s = 0; s < 2; ++s) {
+            add(C.psi[a][s][C.par], L.psi[a][s][L.par], (size_t)P->psi_elems[a] * P->nshots * P->esize);
+            add(C.xi[a][s][0], L.xi[a][s][0], (size_t)P->xi_elems[a] * P->nshots * P->esize);
+        }
+    while (!todo.empty()) {
+        // one whose target nothing else has to leave first; where there is
+        // none (fields in a cycle: every other one is in place), one goes to
+        // the field that has no role in L
+        size_t q = 0;
+        auto blocked = [&](const Move& m) {
+            return std::any_of(todo.begin(), todo.end(), [&](const Move& o) { return o.from == m.to; });
+        };
+        while (q < todo.size() && blocked(todo[q])) ++q;
+        Move& m = todo[q < todo.size() ? q : 0];
+        void* to = q < todo.size() ? m.to : L.p[3];
+        if (!to) return fail(AWCPML_ERR_STATE, "no free field buffer");
+        HIP_TRY(hipMemcpyAsync(to, m.from, m.bytes, hipMemcpyDeviceToDevice, P->stream));
+        if (q < todo.size()) todo.erase(todo.begin() + q);
+        else m.from = to;
+    }
+    HIP_TRY(hipStreamSynchronize(P->stream));
+    set_layout(P, L);
+    return AWCPML_OK;
+}
+
+// A plan whose launches the library chooses may have traded buffers while it
+// ran alone, to the batch's own step: its state goes where the batch has it.
+int batch_settle(awcpml_batch* B) {
+    for (auto* P : B->plans) {
+        if (!P->tb_auto || P->uncounted % 6 || P->it != std::min(B->it, P->nt)) continue;
+        const int st = settle(P, roles_layout(P, B->roles[B->cur].r, P->it));
+        if (st) return st;
+    }
+    return AWCPML_OK;
+}
+
 // After the batch ran to step B->it, every plan is at min(it, its nt), in
 // the batch's roles (which change only while every plan runs).
 void batch_sync_plans(awcpml_batch* B) {
     for (auto* P : B->plans) {
         P->it = std::min(B->it, P->nt);
+        P->uncounted = 0;
         set_layout(P, roles_layout(P, B->roles[B->cur].r, P->it));
     }
 }
@@ -2028,6 +2083,7 @@ int awcpml_reset(awcpml_plan* P) {
         HIP_TRY(hipMemsetAsync(P->d_traces, 0, (size_t)P->n_rec_total * P->nt * P->esize, P->stream));
     HIP_TRY(hipStreamSynchronize(P->stream));
     P->it = 0;
+    P->uncounted = 0;
     P->rot = 0;
     P->par = 0;
     return AWCPML_OK;
@@ -2054,6 +2110,7 @@ int awcpml_forward(awcpml_plan* P, int64_t it) {
     if ((st = ready(P))) return st;
     if (it < 1 || it > P->nt) return fail(AWCPML_ERR_ARG, "it %lld outside 1..nt", (long long)it);
     if ((st = do_step(P, it - 1))) return st;
+    P->uncounted = (P->uncounted + 1) % 6;
     HIP_TRY(hipStreamSynchronize(P->stream));
     return AWCPML_OK;
 }
@@ -2113,6 +2170,7 @@ int awcpml_time_stencil(awcpml_plan* P, int nlaunches, double* ms_total) {
     HIP_TRY(hipEventRecord(e0, P->stream));
     for (int q = 0; q < nlaunches; ++q) {
         if ((st = launch_stencil(P))) break;
+        P->uncounted = (P->uncounted + 1) % 6;
         P->rot = (P->rot + 1) % 3;
         P->par ^= 1;
     }
@@ -2381,6 +2439,8 @@ int awcpml_batch_advance(awcpml_batch* B, int64_t nsteps) {
     if (!B) return fail(AWCPML_ERR_ARG, "batch is NULL");
     if (nsteps < 0) return fail(AWCPML_ERR_ARG, "nsteps < 0");
     if (batch_stale(B)) return batch_stale_error();
+    int st = batch_settle(B);
+    if (st) return st;
     for (auto* P : B->plans)
         if (P->it != std::min(B->it, P->nt) ||
             !(get_layout(P) == roles_layout(P, B->roles[B->cur].r, P->it)))
@@ -2389,7 +2449,7 @@ int awcpml_batch_advance(awcpml_batch* B, int64_t nsteps) {
     if (B->it + nsteps > B->nt_max)
         return fail(AWCPML_ERR_STATE, "advance past the longest run: %lld + %lld > %lld",
                     (long long)B->it, (long long)nsteps, (long long)B->nt_max);
-    int st = batch_run_steps(B, nsteps);
+    st = batch_run_steps(B, nsteps);
     if (!st) {
         hipError_t e = hipStreamSynchronize(B->stream);
         if (e != hipSuccess) st = fail(AWCPML_ERR_HIP, "hipStreamSynchronize failed: %s", hipGetErrorString(e));
@@ -2411,7 +2471,8 @@ int awcpml_batch_time_advance(awcpml_batch* B, int64_t nsteps, double* ms_total)
     if (!B || !ms_total || nsteps < 0) return fail(AWCPML_ERR_ARG, "bad argument");
     if (batch_stale(B)) return batch_stale_error();
     if (B->it + nsteps > B->nt_max) return fail(AWCPML_ERR_STATE, "advance past the longest run");
-    int st;
+    int st = batch_settle(B);
+    if (st) return st;
     if (nsteps > 0 && B->use_graph) {  // capture outside the timed region
         GraphEntry* g = nullptr;
         if ((st = batch_graph(B, nsteps, &g))) return st;
@@ -2672,6 +2733,7 @@ int ck_copy(awcpml_plan* P, int64_t c, bool save) {
         P->rot = P->ck_rot[c];
         P->par = P->ck_par[c];
         P->it = c * P->ck_every;
+        P->uncounted = 0;
     }
     for (int b = 0; b < L.fields; ++b) mv(P->p[(P->rot + b) % 3], L.field);
     for (int a = 0; a < P->ndim; ++a)

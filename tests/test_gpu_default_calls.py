@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import awcpml
+from awcpml import _lib
 from cases import small2d, small3d
 from test_gpu_two_step import _batch_state, _oracle, _plan, _same, _state
 
@@ -75,5 +76,47 @@ def test_batch_goes_on_after_a_plan_ran_on_its_own(nd, own):
         B.set_time_block(2)
         B.run()
         _same(_batch_state(plans), _batch_state(ref))
+    for P in plans + ref:
+        P.close()
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("at", [2, 9, 10, 11, 17])
+def test_batch_takes_a_plan_that_came_to_its_step_alone(nd, at, dtype):
+    """A plan reset and run alone to the batch's step rejoins it there."""
+    print("[gpu] batch takes a plan run alone to step %d, %dD %s" % (at, nd, dtype), flush=True)
+    os_ = [_oracle(_case(nd, nt)) for nt in (30, 26)]
+    ref = [_plan(o, dtype=dtype) for o in os_]
+    for P, o in zip(ref, os_):
+        P.set_time_block(1)
+        P.advance(o.nt)
+    plans = [_plan(o, dtype=dtype) for o in os_]
+    with awcpml.Batch(plans) as B:
+        for graph in (False, True):
+            B.set_graph(graph)
+            B.reset()
+            B.advance(at)
+            plans[0].reset()
+            plans[0].advance(at)
+            if graph:
+                assert B.time_advance(30 - at) > 0
+            else:
+                B.advance(30 - at)
+            _same(_batch_state(plans), _batch_state(ref))
+        # another step than the batch's, and one more beside it, are refused as ever
+        B.reset()
+        B.advance(at)
+        plans[0].reset()
+        plans[0].advance(at)
+        plans[0].forward(1)
+        with pytest.raises(_lib.AwcpmlError, match="stepped or changed on its own"):
+            B.advance(1)
+        B.reset()
+        B.advance(at)
+        plans[0].reset()
+        plans[0].advance(at - 1)
+        with pytest.raises(_lib.AwcpmlError, match="stepped or changed on its own"):
+            B.advance(1)
     for P in plans + ref:
         P.close()
