@@ -2191,8 +2191,9 @@ int awcpml_time_advance(awcpml_plan* P, int64_t nsteps, double* ms_total) {
     if (!ms_total || nsteps < 0) return fail(AWCPML_ERR_ARG, "bad argument");
     if ((st = ready(P))) return st;
     if (P->it + nsteps > P->nt) return fail(AWCPML_ERR_STATE, "advance past nt");
+    // allocation and capture outside the timed region
+    if ((st = auto_spares(P, nsteps))) return st;
     if (P->use_graph && nsteps > 0) {
-        // capture outside the timed region
         GraphEntry* g = nullptr;
         if ((st = plan_graph(P, nsteps, &g))) return st;
     }

@@ -120,3 +120,25 @@ def test_batch_takes_a_plan_that_came_to_its_step_alone(nd, at, dtype):
             B.advance(1)
     for P in plans + ref:
         P.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_first_timed_run_holds_no_allocation(graph):
+    """time_advance of a plan that has not run yet: the buffers it gets (30 MB
+    here) and the graph it captures come before the events, so that a first run
+    of one launch takes what the later ones take."""
+    print("[gpu] first timed run, graph %s" % graph, flush=True)
+    o = _oracle(_case(2, nt=8, n=(300, 290)))
+    first, later = [], []
+    for _ in range(6):
+        P = _plan(o, nshots=44, srcs=[o.positions()[0]] * 44)
+        P.set_graph(graph)
+        P.reset()
+        first.append(P.time_advance(o.nt))
+        assert P.time_block()[0] == 2
+        for _ in range(3):
+            P.reset()
+            later.append(P.time_advance(o.nt))
+        P.close()
+    print(first, later, flush=True)
+    assert min(first) < 1.15 * max(later)
