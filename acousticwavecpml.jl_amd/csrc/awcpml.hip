@@ -2318,7 +2318,8 @@ int awcpml_time_stencil2(awcpml_plan* P, int nlaunches, double* ms_total) {
     if (st) return st;
     if (!ms_total || nlaunches < 1) return fail(AWCPML_ERR_ARG, "bad argument");
     if ((st = ready(P))) return st;
-    if (!two_ok(P)) return fail(AWCPML_ERR_STATE, "two-step launches do not apply to this plan");
+    if (P->time_block != 2 || !two_applies(P))
+        return fail(AWCPML_ERR_STATE, "two-step launches do not apply to this plan (see awcpml_set_time_block)");
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));

@@ -200,7 +200,8 @@ int awcpml_set_two_step_align(awcpml_plan *plan, int enable);
 int awcpml_get_two_step_align(const awcpml_plan *plan, int *enable);
 
 /* Time `nlaunches` two-step stencil launches alone (no source or receiver
- * work), in milliseconds; fails unless two-step launches apply.  The state
+ * work), in milliseconds; fails unless awcpml_set_time_block asked for two
+ * steps and two-step launches apply.  The state
  * advances without sources; call awcpml_reset afterwards.  Measurement
  * support, no reference counterpart. */
 int awcpml_time_stencil2(awcpml_plan *plan, int nlaunches, double *ms_total);

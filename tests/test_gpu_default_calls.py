@@ -142,3 +142,19 @@ def test_first_timed_run_holds_no_allocation(graph):
         P.close()
     print(first, later, flush=True)
     assert min(first) < 1.15 * max(later)
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+def test_stencil2_timing_needs_the_request(nd):
+    """time_stencil2 stays refused for a plan that never asked for two steps."""
+    print("[gpu] time_stencil2 without a request %dD" % nd, flush=True)
+    o = _oracle(_case(nd))
+    P = _plan(o)
+    for ran in (False, True):
+        with pytest.raises(_lib.AwcpmlError, match="do not apply"):
+            P.time_stencil2(1)
+        P.advance(8)
+    P.set_time_block(2)
+    P.reset()
+    assert P.time_stencil2(2) > 0
+    P.close()
