@@ -223,7 +223,8 @@ class Plan:
         return ms.value
 
     def time_stencil2(self, nlaunches):
-        """Milliseconds of `nlaunches` two-step stencil launches."""
+        """Milliseconds of `nlaunches` two-step stencil launches (2D: of as
+        many steps in the longer launches that advance makes)."""
         ms = ctypes.c_double()
         _lib.check(_lib.load().awcpml_time_stencil2(self._h, int(nlaunches), ctypes.byref(ms)))
         return ms.value

@@ -2324,14 +2324,16 @@ int awcpml_time_stencil2(awcpml_plan* P, int nlaunches, double* ms_total) {
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, P->stream));
-    for (int q = 0; q < nlaunches; ++q) {
-        const bool f64 = P->dtype == AWCPML_F64;
+    const bool f64 = P->dtype == AWCPML_F64;
+    for (int64_t left = 2 * (int64_t)nlaunches; left > 0;) {
+        const int n = P->ndim == 2 ? tile_steps(left, false) : 2;
         if (P->ndim == 2)
-            st = f64 ? launch_tile_t<double>(P, 0, 2, nullptr, false) : launch_tile_t<float>(P, 0, 2, nullptr, false);
+            st = f64 ? launch_tile_t<double>(P, 0, n, nullptr, false) : launch_tile_t<float>(P, 0, n, nullptr, false);
         else
             st = f64 ? launch_stencil2_t<double>(P, 0) : launch_stencil2_t<float>(P, 0);
         if (st) break;
         two_swap(P);
+        left -= n;
     }
     HIP_TRY(hipEventRecord(e1, P->stream));
     HIP_TRY(hipEventSynchronize(e1));

@@ -158,3 +158,34 @@ def test_stencil2_timing_needs_the_request(nd):
     P.reset()
     assert P.time_stencil2(2) > 0
     P.close()
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_2d_stencil_timing_is_of_the_launches_that_run(dtype):
+    """time_stencil2 of a 2D plan times its steps in launches as long as
+    awcpml_advance makes them.  One source and a few receivers add little to
+    44 shots of 300 x 290 nodes, so both agree within half (a launch of two
+    steps takes three times as long per step)."""
+    print("[gpu] 2D stencil timing %s" % dtype, flush=True)
+    o = _oracle(_case(2, nt=160, n=(300, 290)))
+    P = _plan(o, dtype=dtype, nshots=44, srcs=[o.positions()[0]] * 44)
+    P.set_time_block(2)
+    stencil, run = [], []
+    for _ in range(4):
+        P.reset()
+        run.append(P.time_advance(160) / 160)
+        P.reset()
+        stencil.append(P.time_stencil2(80) / 160)
+    print(stencil, run, flush=True)
+    assert 0.5 < min(stencil) / min(run) < 1.5
+    for n in (1, 2, 3):
+        P.reset()
+        assert P.time_stencil2(n) > 0
+    P.reset()
+    P.advance(o.nt)
+    two = _state(P, 1)
+    P.set_time_block(1)
+    P.reset()
+    P.advance(o.nt)
+    _same(two, _state(P, 1))
+    P.close()
