@@ -2993,7 +2993,8 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     io.ndim = P->ndim;
     io.rq = (T*)Bf.rq;
 
-    const bool wide = (uint64_t)P->field_elems * sizeof(T) >= (1ull << 32);  // byte offsets past 32 bits
+    // byte offsets past 32 bits
+    const bool wide = P->wide || (uint64_t)P->field_elems * sizeof(T) >= (1ull << 32);
     int lr = 0, par = 0;
     for (int64_t seg = P->ck_count - 1; seg >= 0; --seg) {
         const int64_t c0 = seg * K, c1 = std::min<int64_t>(c0 + K, nt);

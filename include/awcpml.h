@@ -206,7 +206,8 @@ int awcpml_get_two_step_align(const awcpml_plan *plan, int *enable);
  * support, no reference counterpart. */
 int awcpml_time_stencil2(awcpml_plan *plan, int nlaunches, double *ms_total);
 
-/* Force the kernels' 64-bit address offsets on any grid (enable != 0).
+/* Force the kernels' 64-bit address offsets on any grid (enable != 0),
+ * those of awcpml_adjoint's reverse step too.
  * The library switches to them by itself for fields of 4 GiB and more per
  * shot; results are bit-identical either way.  Two-step launches do not
  * apply to such plans (they take single steps).  Test support for the

@@ -189,3 +189,24 @@ def test_2d_stencil_timing_is_of_the_launches_that_run(dtype):
     P.advance(o.nt)
     _same(two, _state(P, 1))
     P.close()
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n,shots", [((70, 61), 3), ((40, 37), 5), ((30, 26, 24), 2), ((66, 17, 15), 5)])
+def test_gradient_with_wide_offsets(n, shots, dtype):
+    """The reverse step with 64-bit offsets (fields of 4 GiB and more per shot)
+    forced on small grids: bitwise the 32-bit one."""
+    print("[gpu] gradient with wide offsets %s %s" % (n, dtype), flush=True)
+    o = _oracle(_case(len(n), nt=110, n=n))
+    o.run()
+    obs = [0.5 * o.traces()] * shots
+    P = _plan(o, dtype=dtype, nshots=shots, srcs=[o.positions()[0]] * shots)
+    for group in (0, 1, 2):
+        P.set_adjoint_group(group)
+        P.set_wide_offsets(False)
+        J, g = awcpml.fwi.misfit_gradient(P, obs, every=7)
+        P.set_wide_offsets(True)
+        Jw, gw = awcpml.fwi.misfit_gradient(P, obs, every=7)
+        assert P.time_block()[0] == 1
+        assert J == Jw and np.array_equal(g, gw) and np.abs(g).max() > 0
+    P.close()
