@@ -199,7 +199,7 @@ struct awcpml_plan {
     // spare buffers, which then trade places with the buffers they replace
     int time_block = 1;
     bool tb_auto = true;             // awcpml_set_time_block was not called: the library decides
-    bool spare_failed = false;       // ... and the spare buffers did not fit
+    bool spare_failed = false;       // ... and the spare buffers did not fit since the last reset
     int tb_rows = 0, tb_march = 0;   // waves per block, chunk length (0: default)
     // 3D: two_shape's choice for the current CPML sides and tb_rows; 0: none yet
     mutable int two_rows = 0, two_march = 0;
@@ -1267,7 +1267,9 @@ constexpr size_t kAskFreeBytes = 64ull << 20;
 // A plan left to the library's choice gets its spare buffers with its first
 // run of several steps; where they do not fit, or would take more than an
 // eighth of the device memory that is free (which the caller may count on; not
-// counting `later` bytes the library is about to need), it keeps single steps.
+// counting `later` bytes the library is about to need), it keeps single steps
+// until the next reset, after which the question is open again.  A gradient's
+// `later` bytes bind no other run.
 int auto_spares(awcpml_plan* P, int64_t n, size_t later = 0) {
     if (!P->tb_auto || n < 2 || P->p_spare || P->spare_failed || !multi_possible(P)) return AWCPML_OK;
     int64_t elems = P->field_elems;
@@ -1277,7 +1279,7 @@ int auto_spares(awcpml_plan* P, int64_t n, size_t later = 0) {
     if (bytes + later > kAskFreeBytes) {
         HIP_TRY(hipMemGetInfo(&avail, &total));
         if (bytes > (avail - std::min(avail, later)) / 8) {
-            P->spare_failed = true;
+            P->spare_failed = later == 0;
             return AWCPML_OK;
         }
     }
@@ -2079,6 +2081,7 @@ int awcpml_reset(awcpml_plan* P) {
             }
         }
     P->boundary_dirty = false;
+    P->spare_failed = false;
     if (P->d_traces && P->n_rec_total > 0 && P->nt > 0)
         HIP_TRY(hipMemsetAsync(P->d_traces, 0, (size_t)P->n_rec_total * P->nt * P->esize, P->stream));
     HIP_TRY(hipStreamSynchronize(P->stream));

@@ -6,6 +6,8 @@ runs, memory that has run short).
 Everything is compared value for value with a plan set to single steps, or with
 the same call made another way.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -209,4 +211,64 @@ def test_gradient_with_wide_offsets(n, shots, dtype):
         Jw, gw = awcpml.fwi.misfit_gradient(P, obs, every=7)
         assert P.time_block()[0] == 1
         assert J == Jw and np.array_equal(g, gw) and np.abs(g).max() > 0
+    P.close()
+
+
+class _Ballast:
+    """Device memory taken so that `left` bytes stay free."""
+
+    def __init__(self, left):
+        self.hip = ctypes.CDLL("libamdhip64.so.7")
+        self.hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+        self.hip.hipFree.argtypes = [ctypes.c_void_p]
+        self.ptrs = []
+        while self.free() > left:
+            p = ctypes.c_void_p()
+            assert self.hip.hipMalloc(ctypes.byref(p), min(self.free() - left, 32 << 30)) == 0
+            self.ptrs.append(p)
+
+    def free(self):
+        v, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert self.hip.hipMemGetInfo(ctypes.byref(v), ctypes.byref(t)) == 0
+        return v.value
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        for p in self.ptrs:
+            self.hip.hipFree(p)
+
+
+def test_spares_refused_once_are_asked_for_again():
+    """A gradient's forward run that keeps single steps for the memory its
+    reverse steps would need (here 336 GB) does not bind the runs after it."""
+    print("[gpu] spares after a refusal", flush=True)
+    K = 25000
+    o = _oracle(_case(3, nt=K, n=(160, 150, 140)))
+    P = _plan(o, dtype="f32")
+    P.checkpoint_run(K)
+    assert P.time_block()[0] == 1
+    P.reset()
+    P.advance(6)
+    assert P.time_block()[0] == 2
+    P.close()
+
+
+def test_spares_refused_for_lack_of_memory_come_with_the_next_reset():
+    """Little free memory at one run does not bind the runs after a reset."""
+    print("[gpu] spares after a shortage", flush=True)
+    n, S = (128, 160, 160), 10
+    o = _oracle(_case(3, nt=9, n=n))
+    P = _plan(o, dtype="f32", nshots=S, srcs=[o.positions()[0]] * S)
+    with _Ballast(4 * S * int(np.prod(n)) * 7):  # less than 8 times the spare field
+        P.advance(4)
+        assert P.time_block()[0] == 1
+    P.advance(5)
+    assert P.time_block()[0] == 1
+    one = _state(P, 1)
+    P.reset()
+    P.advance(9)
+    assert P.time_block()[0] == 2
+    _same(_state(P, 1), one)
     P.close()
