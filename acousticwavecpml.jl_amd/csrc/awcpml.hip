@@ -1401,6 +1401,7 @@ struct awcpml_batch {
     std::vector<RoleTables> roles;   // built on first use, kept until destroy
     int cur = 0;                     // roles[cur]: the plans' roles now
     int time_block = 1, tb_rows = 0, tb_prefetch = 0;
+    int two_march = 0;               // chunk length of 3D plans that set none; 0: none yet
     std::vector<int> block_start, block_start2, shot_start;
     int grid_blocks = 0, grid_blocks2 = 0;
     int64_t it = 0, nt_max = 0, nt_min = 0;
@@ -1428,13 +1429,14 @@ bool batch_two_ok(const awcpml_batch* B) {
 template <typename T>
 int batch_tables_t(awcpml_batch* B, const Roles& R, RoleTables* out) {
     const int np = (int)B->plans.size();
-    bool two = true;
+    bool two = B->time_block == 2;
     for (auto* P : B->plans) two = two && P->p_spare;
     int W, pf;
     batch_two_shape(B, &W, &pf);
-    int common = 0;  // chunk length of the plans that set none
-    if (two && B->ndim == 3)
-        two_shape(std::vector<const awcpml_plan*>(B->plans.begin(), B->plans.end()), W, &W, &common);
+    // one choice for the tables of all roles (187x131x223, 3 shots, and 100^3, 2
+    // shots, FP32, first graph of 64 steps: 8.5 ms with a choice each, 7.8 so)
+    if (two && B->ndim == 3 && B->two_march == 0)
+        two_shape(std::vector<const awcpml_plan*>(B->plans.begin(), B->plans.end()), W, &W, &B->two_march);
     std::vector<StencilArgs<T>> args((size_t)6 * np);
     std::vector<awcpml::Stencil2Args<T>> args2(two ? (size_t)6 * np : 0);
     std::vector<awcpml::IoArgs<T>> io((size_t)6 * np);
@@ -1444,7 +1446,7 @@ int batch_tables_t(awcpml_batch* B, const Roles& R, RoleTables* out) {
         set_layout(P, roles_layout(P, R, 0));
         for (int v = 0; v < 6; ++v) args[(size_t)v * np + q] = make_args<T>(P, v % 3, v % 2);
         if (two) {
-            const int ml = B->ndim == 2 ? march_2d(P) : P->tb_march > 0 ? P->tb_march : common;
+            const int ml = B->ndim == 2 ? march_2d(P) : P->tb_march > 0 ? P->tb_march : B->two_march;
             for (int v = 0; v < 6; ++v) {
                 P->rot = v % 3;
                 P->par = v % 2;
@@ -1524,6 +1526,7 @@ int batch_rebuild(awcpml_batch* B) {
     for (auto& t : B->roles) free_tables(t);
     B->roles.clear();
     B->cur = 0;
+    B->two_march = 0;
     B->gens.clear();
     for (auto* P : B->plans) B->gens.push_back(P->gen);
     return batch_roles(B, R, &B->cur);
