@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -24,6 +25,7 @@
 #include <functional>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "adjoint_kernels.h"
@@ -330,6 +332,25 @@ int group_alloc(BufferGroup& G, GroupList& L) {
     return AWCPML_OK;
 }
 
+int give_back_spares(awcpml_plan* P);
+
+// alloc(), and where it finds no memory while the plan holds spare buffers that
+// nobody asked for, once more without them: what fits beside single steps fits.
+template <typename Alloc>
+int alloc_first(awcpml_plan* P, Alloc alloc) {
+    int st = alloc();
+    if (st != AWCPML_ERR_NOMEM || !P->tb_auto || !P->p_spare) return st;
+    (void)hipGetLastError();
+    if ((st = give_back_spares(P))) return st;
+    // freed memory can be had a little later (0.3 ms for 190 MB)
+    for (int q = 0; q < 50 && (st = alloc()) == AWCPML_ERR_NOMEM; ++q) {
+        (void)hipGetLastError();
+        std::this_thread::sleep_for(std::chrono::milliseconds(1));
+    }
+    if (!st) g_err.clear();
+    return st;
+}
+
 // Staged transfers take at most this many FP64 values at a time (32 MiB per
 // plan; longer arrays go in pieces, in order on the plan's stream).
 constexpr int64_t kStageElems = 4ll << 20;
@@ -350,7 +371,8 @@ int stage_buffer(awcpml_plan* P, int64_t row, int64_t want) {
     }
     for (int64_t n = want;; n = std::max(row, n / 8)) {
         void* v = nullptr;
-        const int st = dalloc(&v, (size_t)n * 8);
+        auto alloc = [&]() { return dalloc(&v, (size_t)n * 8); };
+        const int st = n > row ? alloc() : alloc_first(P, alloc);
         if (!st) {
             P->stage = (double*)v;
             P->stage_elems = n;
@@ -685,7 +707,7 @@ int sync_io(awcpml_plan* P) {
     L.add(&P->d_io_lists, lists.size());
     L.add(&P->d_src_wav, wav.size() * P->esize);
     L.add(&P->d_traces, trace_bytes);
-    int st = group_alloc(P->io, L);
+    int st = alloc_first(P, [&]() { return group_alloc(P->io, L); });
     if (st) return st;
     char* base = (char*)P->d_io_lists;
     P->d_src_lin = base + at_slin;
@@ -1262,6 +1284,71 @@ int alloc_spares(awcpml_plan* P) {
     return AWCPML_OK;
 }
 
+// Move the plan's state into the buffers of layout L (the same buffers in other
+// roles): every field, the current psi, and xi; what the next step overwrites
+// stays where it is.
+int settle(awcpml_plan* P, const BufLayout& L) {
+    const BufLayout C = get_layout(P);
+    if (C == L) return AWCPML_OK;
+    struct Move {
+        void *from, *to;
+        size_t bytes;
+    };
+    std::vector<Move> todo;
+    auto add = [&](void* from, void* to, size_t bytes) {
+        if (from != to && bytes) todo.push_back({from, to, bytes});
+    };
+    for (int b = 0; b < 3; ++b)
+        add(C.p[(C.rot + b) % 3], L.p[(L.rot + b) % 3], (size_t)P->field_elems * P->nshots * P->esize);
+    for (int a = 0; a < P->ndim; ++a)
+        for (int s = 0; s < 2; ++s) {
+            add(C.psi[a][s][C.par], L.psi[a][s][L.par], (size_t)P->psi_elems[a] * P->nshots * P->esize);
+            add(C.xi[a][s][0], L.xi[a][s][0], (size_t)P->xi_elems[a] * P->nshots * P->esize);
+        }
+    while (!todo.empty()) {
+        // one whose target nothing else has to leave first; where there is
+        // none (fields in a cycle: every other one is in place), one goes to
+        // the field that has no role in L
+        size_t q = 0;
+        auto blocked = [&](const Move& m) {
+            return std::any_of(todo.begin(), todo.end(), [&](const Move& o) { return o.from == m.to; });
+        };
+        while (q < todo.size() && blocked(todo[q])) ++q;
+        Move& m = todo[q < todo.size() ? q : 0];
+        void* to = q < todo.size() ? m.to : L.p[3];
+        if (!to) return fail(AWCPML_ERR_STATE, "no free field buffer");
+        HIP_TRY(hipMemcpyAsync(to, m.from, m.bytes, hipMemcpyDeviceToDevice, P->stream));
+        if (q < todo.size()) todo.erase(todo.begin() + q);
+        else m.from = to;
+    }
+    HIP_TRY(hipStreamSynchronize(P->stream));
+    set_layout(P, L);
+    return AWCPML_OK;
+}
+
+// Free the spare buffers the library took for a plan, its state moved into the
+// others; it takes single steps until the next reset.
+int give_back_spares(awcpml_plan* P) {
+    BufLayout L = P->home;
+    L.rot = P->rot;
+    L.par = P->par;
+    const int st = settle(P, L);
+    if (st) return st;
+    drop_graphs(P->graphs);
+    GroupList G;
+    G.add(&P->p_spare, 0);
+    for (int a = 0; a < 3; ++a)
+        for (int s = 0; s < 2; ++s) {
+            G.add(&P->psi_spare[a][s], 0);
+            G.add(&P->xi_spare[a][s], 0);
+            P->home.psi[a][s][2] = P->home.xi[a][s][1] = nullptr;
+        }
+    group_free(P->spares, G);
+    P->home.p[3] = nullptr;
+    P->spare_failed = true;
+    return AWCPML_OK;
+}
+
 constexpr size_t kAskFreeBytes = 64ull << 20;
 
 // A plan left to the library's choice gets its spare buffers with its first
@@ -1709,48 +1796,6 @@ int batch_prepare(awcpml_batch* B, int64_t it0, int64_t n) {
             q += 1;
         }
     }
-    return AWCPML_OK;
-}
-
-// Move the plan's state into the buffers of layout L (the same buffers in other
-// roles): every field, the current psi, and xi; what the next step overwrites
-// stays where it is.
-int settle(awcpml_plan* P, const BufLayout& L) {
-    const BufLayout C = get_layout(P);
-    if (C == L) return AWCPML_OK;
-    struct Move {
-        void *from, *to;
-        size_t bytes;
-    };
-    std::vector<Move> todo;
-    auto add = [&](void* from, void* to, size_t bytes) {
-        if (from != to && bytes) todo.push_back({from, to, bytes});
-    };
-    for (int b = 0; b < 3; ++b)
-        add(C.p[(C.rot + b) % 3], L.p[(L.rot + b) % 3], (size_t)P->field_elems * P->nshots * P->esize);
-    for (int a = 0; a < P->ndim; ++a)
-        for (int s = 0; s < 2; ++s) {
-            add(C.psi[a][s][C.par], L.psi[a][s][L.par], (size_t)P->psi_elems[a] * P->nshots * P->esize);
-            add(C.xi[a][s][0], L.xi[a][s][0], (size_t)P->xi_elems[a] * P->nshots * P->esize);
-        }
-    while (!todo.empty()) {
-        // one whose target nothing else has to leave first; where there is
-        // none (fields in a cycle: every other one is in place), one goes to
-        // the field that has no role in L
-        size_t q = 0;
-        auto blocked = [&](const Move& m) {
-            return std::any_of(todo.begin(), todo.end(), [&](const Move& o) { return o.from == m.to; });
-        };
-        while (q < todo.size() && blocked(todo[q])) ++q;
-        Move& m = todo[q < todo.size() ? q : 0];
-        void* to = q < todo.size() ? m.to : L.p[3];
-        if (!to) return fail(AWCPML_ERR_STATE, "no free field buffer");
-        HIP_TRY(hipMemcpyAsync(to, m.from, m.bytes, hipMemcpyDeviceToDevice, P->stream));
-        if (q < todo.size()) todo.erase(todo.begin() + q);
-        else m.from = to;
-    }
-    HIP_TRY(hipStreamSynchronize(P->stream));
-    set_layout(P, L);
     return AWCPML_OK;
 }
 
@@ -2887,7 +2932,7 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
     const size_t zeros = L.want.size(), zero_bytes = L.total;
     L.add(&Bf.q, fb * (size_t)K);
     L.add(&Bf.tbar, ntr * sizeof(T));
-    if ((st = group_alloc(Bf.main, L))) return st;
+    if ((st = alloc_first(P, [&]() { return group_alloc(Bf.main, L); }))) return st;
     if (Bf.main.base) {
         HIP_TRY(hipMemsetAsync(Bf.main.base, 0, zero_bytes, P->stream));
     } else {
@@ -2976,7 +3021,7 @@ int adjoint_t(awcpml_plan* P, const double* tbar, double* fbar) {
         put(&Bf.rf_idx, rf_idx.data(), rf_idx.size() * 4);
         Bf.want_lists.add(&Bf.list_block, lists.size());
         Bf.want_lists.add(&Bf.rq, node_lin.size() * sizeof(T));
-        if ((st = group_alloc(Bf.lists, Bf.want_lists))) return st;
+        if ((st = alloc_first(P, [&]() { return group_alloc(Bf.lists, Bf.want_lists); }))) return st;
         for (auto& a : at) *a.first = (char*)Bf.list_block + a.second;
         HIP_TRY(hipMemcpyAsync(Bf.list_block, lists.data(), lists.size(), hipMemcpyHostToDevice, P->stream));
         if (rf_count) HIP_TRY(hipMemsetAsync(Bf.rq, 0, node_lin.size() * sizeof(T), P->stream));
@@ -3071,7 +3116,7 @@ int awcpml_checkpoint_run(awcpml_plan* P, int64_t every) {
     if (need > P->ck_alloc) {
         dfree(P->ck);
         P->ck_alloc = 0;
-        if ((st = dalloc(&P->ck, need))) return st;
+        if ((st = alloc_first(P, [&]() { return dalloc(&P->ck, need); }))) return st;
         P->ck_alloc = need;
     }
     P->ck_every = every;

@@ -169,8 +169,9 @@ int awcpml_get_shot_group(const awcpml_plan *plan, int *shot_group);
  * per launch.  steps = 1: one step per launch.  A plan for which this is
  * never called takes launches of several steps where those apply and their
  * spare buffers need at most an eighth of the free device memory (allocated
- * with the first run of two steps or more, and kept; refused, the plan takes
- * single steps, and the first run after the next awcpml_reset asks again).
+ * with the first run of two steps or more, and kept unless the plan itself
+ * needs the memory later; refused or given back, the plan takes single steps,
+ * and the first run after the next awcpml_reset asks again).
  * They are a third more than the three fields and half more than psi and xi:
  * awcpml_set_time_block(plan, 1, 0, 0, 0) before the first run saves them,
  * awcpml_get_time_block after it tells.

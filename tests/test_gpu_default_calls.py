@@ -272,3 +272,37 @@ def test_spares_refused_for_lack_of_memory_come_with_the_next_reset():
     assert P.time_block()[0] == 2
     _same(_state(P, 1), one)
     P.close()
+
+
+def test_gradient_takes_the_spares_memory_back():
+    """A gradient that fits only without the spare buffers the library took for
+    an earlier run still fits."""
+    print("[gpu] gradient in the memory of the spares", flush=True)
+    n, K, S, h = (128, 160, 160), 10, 10, 5
+    case = _case(3, nt=K, n=n, freetop=False)
+    case["recpos"] = case["srcpos"] + np.array([[0.0] * 3, [20.0, 10.0, 0.0]])
+    o = _oracle(case)
+    P = _plan(o, dtype="f32", nshots=S, srcs=[o.positions()[0]] * S)
+    P.set_adjoint_group(S)
+    tbar = [np.ones((K, P._nrecs[s])) for s in range(S)]
+    P.checkpoint_run(K)
+    assert P.time_block()[0] == 2
+    want = P.adjoint(tbar)
+    assert np.abs(want).max() > 0
+    fields = _state(P, S)
+    # K fields of q, 3 of lam, two sets of slabs, the accumulators
+    N = int(np.prod(n))
+    slabs = sum((2 * h + 1) * N // v for v in n)
+    need = 4 * S * (N * (K + 3) + 4 * slabs) + 12 * N
+    spares = 4 * S * (N + 2 * slabs)
+    P.checkpoint_run(K)
+    with _Ballast(need - spares // 2) as B:
+        print("[gpu] free %d of %d needed" % (B.free(), need), flush=True)
+        got = P.adjoint(tbar)
+    assert P.time_block()[0] == 1
+    assert np.array_equal(got, want)
+    _same(_state(P, S), fields)
+    P.reset()
+    P.advance(K)
+    assert P.time_block()[0] == 2
+    P.close()
