@@ -14,7 +14,9 @@ rows of several shots, sharing the model rows they read).  Two-step
 launches (``Plan.set_time_block``: two time steps per launch, bit-identical
 results) are timed per time step too, each shape with aligned 64-node x
 tiles and with 62-node tiles (``Plan.set_two_step_align``), and kept when
-they are faster; the choice is recorded as ``time_block["align"]``.
+they are faster; the choice is recorded as ``time_block["align"]``.  2D
+plans, whose launches of up to eight steps have one shape, compare whole
+steps with sources and receivers (``ms_per_whole_step``).
 """
 import json
 import os
@@ -136,11 +138,20 @@ def autotune(plan, cands=None, launches=8, cache=DEFAULT_CACHE, use_cache=True):
     if plan.ndim == 2 and cands is None and plan.nt:
         # 2D launches of several steps have one shape and handle sources and
         # receivers themselves: whole steps are compared
-        single = _ms_per_step(plan)
-        plan.set_time_block(2)
-        multi = _ms_per_step(plan)
-        if multi < single:
-            two.append((best["ms_per_step"] * multi / single, 0, 0, 0, None))
+        single = best["ms_per_whole_step"] = _ms_per_step(plan)
+        try:
+            plan.set_time_block(2)
+            multi = _ms_per_step(plan)
+            # (equal runs where launches of several steps do not apply)
+            if plan.time_block()[0] == 2:
+                best["tried"] += 1
+                if multi < single:
+                    n2 = 4 * max(1, launches // 2)  # 2 * n2 steps, eight a launch
+                    best["ms_per_step"] = plan.time_stencil2(n2) / n2 / 2.0
+                    best["ms_per_whole_step"] = multi
+                    best["time_block"] = {"block_rows": 0, "march_len": 0, "prefetch": 0}
+        except _lib.AwcpmlError:
+            pass  # the spare buffers do not fit: single steps
     for w, ml2, pf2 in (two_step_candidates(plan) if cands is None and plan.ndim == 3 else []):
         try:
             for al in aligns:

@@ -1,0 +1,64 @@
+"""CPU tests of the autotuner's 2D branch and cache, with the stand-in plan of
+test_autotune_host: launches of several steps are taken where they apply and are
+faster, and single steps kept where their buffers do not fit."""
+import pytest
+
+from awcpml import _lib
+from test_autotune_host import FakePlan, at
+
+
+class Fake2D(FakePlan):
+    """Whole steps of `one` ms, of `multi` ms in launches of several steps."""
+
+    def __init__(self, one=1.0, multi=0.3, applies=True, fits=True):
+        super().__init__(ndim=2)
+        self.nt, self.one, self.multi, self.applies, self.fits = 100, one, multi, applies, fits
+
+    def set_time_block(self, steps, *shape):
+        if steps == 2 and not self.fits:
+            raise _lib.AwcpmlError(-3, "out of memory")
+        super().set_time_block(steps, *shape)
+
+    def time_block(self):
+        return (2 if self.tb[0] == 2 and self.applies else 1, 4, 16, 2)
+
+    def advance(self, n):
+        pass
+
+    def time_advance(self, n):
+        return n * (self.multi if self.tb[0] == 2 else self.one)
+
+    def time_stencil2(self, n):
+        return 0.25 * 2 * n
+
+
+def test_2d_takes_several_steps_per_launch(tmp_path):
+    P = Fake2D()
+    best = at.autotune(P, cache=str(tmp_path / "t.json"))
+    assert P.tb[0] == 2 and best["time_block"] is not None
+    # both figures are measured: whole steps, and the stencil launches alone
+    assert best["ms_per_whole_step"] == pytest.approx(0.3)
+    assert best["ms_per_step"] == pytest.approx(0.25)
+    Q = Fake2D()
+    assert at.autotune(Q, cache=str(tmp_path / "t.json"))["cached"] and Q.tb[0] == 2
+
+
+def test_2d_keeps_single_steps_when_faster(tmp_path):
+    P = Fake2D(multi=1.2)
+    best = at.autotune(P, cache=str(tmp_path / "t.json"))
+    assert P.tb[0] == 1 and best["time_block"] is None
+    assert best["ms_per_whole_step"] == pytest.approx(1.0)
+    assert best["ms_per_step"] == best["ms_per_launch"]
+
+
+def test_2d_buffers_that_do_not_fit(tmp_path):
+    P = Fake2D(fits=False)
+    best = at.autotune(P, cache=str(tmp_path / "t.json"))
+    assert P.tb[0] == 1 and best["time_block"] is None
+
+
+def test_2d_launches_that_do_not_apply(tmp_path):
+    """Two identical single-step runs: the second one's luck decides nothing."""
+    P = Fake2D(multi=0.99, applies=False)
+    best = at.autotune(P, cache=str(tmp_path / "t.json"))
+    assert P.tb[0] == 1 and best["time_block"] is None
