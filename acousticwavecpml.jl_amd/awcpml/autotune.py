@@ -3,8 +3,8 @@
 For a plan, time each candidate (block_y, march_len, prefetch, shot_group) with HIP
 events around a few stencil launches (``Plan.time_stencil``), keep the
 fastest, apply it to the plan and remember it in a JSON cache keyed by the
-problem's shape, halo, precision and shot count.  The wavefield state is
-reset afterwards.
+problem's shape, halo, precision and shot count and by the kernels' sources.
+The wavefield state is reset afterwards.
 
     from awcpml.autotune import autotune
     best = autotune(plan)            # {"block_y": 4, "march_len": 148, ...}
@@ -18,6 +18,8 @@ they are faster; the choice is recorded as ``time_block["align"]``.  2D
 plans, whose launches of up to eight steps have one shape, compare whole
 steps with sources and receivers (``ms_per_whole_step``).
 """
+import functools
+import hashlib
 import json
 import os
 
@@ -79,9 +81,26 @@ def _apply(plan, best):
         plan.set_time_block(1)
 
 
+@functools.lru_cache(maxsize=None)
+def _kernels():
+    """Digest of the kernel and host sources (of the library, where they are
+    not there): a choice timed with other kernels or defaults is timed anew."""
+    from . import _lib
+    csrc = os.path.join(_lib.PKG_ROOT, "csrc")
+    files = sorted(os.path.join(csrc, f) for f in os.listdir(csrc)) if os.path.isdir(csrc) else []
+    digest = hashlib.sha1()
+    for path in files or [_lib.LIB_PATH]:
+        try:
+            with open(path, "rb") as fh:
+                digest.update(fh.read())
+        except OSError:
+            pass
+    return digest.hexdigest()[:12]
+
+
 def _key(plan):
-    return "%dD:%s:h%d:%s:s%d" % (plan.ndim, "x".join(map(str, plan.n)), plan.halo,
-                                   "f64" if plan.dtype == 0 else "f32", plan.nshots)
+    return "%dD:%s:h%d:%s:s%d:%s" % (plan.ndim, "x".join(map(str, plan.n)), plan.halo,
+                                      "f64" if plan.dtype == 0 else "f32", plan.nshots, _kernels())
 
 
 def _load(path):

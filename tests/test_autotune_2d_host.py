@@ -1,6 +1,9 @@
 """CPU tests of the autotuner's 2D branch and cache, with the stand-in plan of
 test_autotune_host: launches of several steps are taken where they apply and are
-faster, and single steps kept where their buffers do not fit."""
+faster, and single steps kept where their buffers do not fit.  Choices that
+other kernels were timed for do not count."""
+import json
+
 import pytest
 
 from awcpml import _lib
@@ -62,3 +65,19 @@ def test_2d_launches_that_do_not_apply(tmp_path):
     P = Fake2D(multi=0.99, applies=False)
     best = at.autotune(P, cache=str(tmp_path / "t.json"))
     assert P.tb[0] == 1 and best["time_block"] is None
+
+
+def test_choices_of_other_kernels_are_timed_anew(tmp_path):
+    """An entry without the kernels' digest, or with another, would pin the plan
+    to a choice that the present kernels were not timed for."""
+    old = {"block_y": 4, "march_len": 64, "prefetch": 3, "shot_group": 1, "ms_per_launch": 1.0,
+           "ms_per_step": 1.0, "time_block": None, "tried": 3}
+    P = Fake2D()
+    plain = "2D:298x298:h20:f32:s8"
+    assert at._key(P).startswith(plain + ":")
+    cache = tmp_path / "old.json"
+    cache.write_text(json.dumps({plain: old, plain + ":0123456789ab": old}))
+    best = at.autotune(P, cache=str(cache))
+    assert not best["cached"] and P.tb[0] == 2
+    assert set(json.loads(cache.read_text())) == {plain, plain + ":0123456789ab", at._key(P)}
+    assert at.autotune(Fake2D(), cache=str(cache))["cached"]
