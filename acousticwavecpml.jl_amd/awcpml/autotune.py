@@ -45,9 +45,11 @@ def candidates(plan):
 
 
 def two_step_candidates(plan):
-    """(block_rows, march_len, prefetch) of 3D two-step launches worth timing."""
+    """(block_rows, march_len, prefetch) of 3D two-step launches worth timing;
+    (0, 0, 0) is the library's choice, so that a tuned plan is no slower than
+    an untuned one."""
     n_march = plan.n[2] - 2
-    out = []
+    out = [(0, 0, 0)]
     for w in ((16, 8) if plan.dtype != 0 else (8, 4)):
         # FP64 on 298^3 (8 waves): chunk 40 measured 3 % faster than 48
         lens = (24, 48, 96, 144) if w == 16 else (24, 32, 40, 48, 96)

@@ -1,4 +1,5 @@
-"""CPU tests of the autotuner's 2D branch and cache, with the stand-in plan of
+"""CPU tests of the autotuner's 2D branch, its cache and the library's own 3D
+choice, with the stand-in plan of
 test_autotune_host: launches of several steps are taken where they apply and are
 faster, and single steps kept where their buffers do not fit.  Choices that
 other kernels were timed for do not count."""
@@ -81,3 +82,14 @@ def test_choices_of_other_kernels_are_timed_anew(tmp_path):
     assert not best["cached"] and P.tb[0] == 2
     assert set(json.loads(cache.read_text())) == {plain, plain + ":0123456789ab", at._key(P)}
     assert at.autotune(Fake2D(), cache=str(cache))["cached"]
+
+
+def test_3d_library_choice_is_a_candidate(tmp_path):
+    cache = str(tmp_path / "t.json")
+    ms = {(0, 0, 0, True): 1.3, (0, 0, 0, False): 1.5, (16, 144, 3, True): 1.4}
+    P = FakePlan(two_ms=ms, one_ms=0.95)
+    best = at.autotune(P, cache=cache)
+    assert P.tb == (2, 0, 0, 0) and P.align is True
+    assert best["time_block"] == {"block_rows": 0, "march_len": 0, "prefetch": 0, "align": True}
+    Q = FakePlan(two_ms=ms, one_ms=0.95)
+    assert at.autotune(Q, cache=cache)["cached"] and Q.tb == (2, 0, 0, 0)
