@@ -826,7 +826,10 @@ int two_chunk_list(const awcpml_plan* P, int ml, int* starts) {
 // On 39 grids and shot counts from 30x32x28 to 450x430x300 nodes, every shape
 // timed, this is 1.4 % above the best shape on average and 19 % at worst; a fixed
 // target of 2048 blocks of 16 to 128 planes is up to 40 % above it (a batch of
-// 170^3, 234^3 and 298^3: FP32 233 and 216 us per step, FP64 497 and 445).
+// 170^3, 234^3 and 298^3: FP32 233 and 216 us per step, FP64 497 and 445).  The
+// rule for FP64 rests on the four grids named.  Longer chunks and more planes
+// ahead are left to timing: 298^3, 8 shots, FP32, 144 planes with 3 ahead take
+// 1.446 ms per launch, the choice made here 1.465.
 void two_shape(const std::vector<const awcpml_plan*>& plans, int rows, int* rows_out, int* march) {
     const bool f64 = plans[0]->dtype == AWCPML_F64;
     const bool even = plans.size() == 1 && plans[0]->nshots % 4 == 0;

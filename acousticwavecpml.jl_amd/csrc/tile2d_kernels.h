@@ -18,11 +18,15 @@
 // through an LDS copy of the tile, made only in blocks that have receivers.
 // So a launch replaces n stencil and n source/receiver launches.
 //
-// Measured (MI355X, whole passes, before -> after): 1066^2 x 64 shots FP32,
-// 182 -> 84 us per step (HBM: the tiles' loads and stores move 1.7 GB per
-// launch of the plain tiles at 5.2 TB/s; the slab tiles are VALU-bound);
-// 298^2 FP64, one shot, 10.8 -> 2.1 us per step (latency: 133 blocks);
-// 4097^2 FP64, 102 -> 28 us per step; 701x333 FP32, 7 shots, 15 -> 4.5 us.
+// Measured (MI355X, HIP events around runs of 200 to 1000 steps with sources and
+// receivers, single steps -> tiles): 1066^2 x 64 shots FP32, 238 -> 71 us per
+// step; 298^2 FP64, one shot, 15.7 -> 2.1 us (latency: 133 blocks); 4097^2 FP64,
+// 133 -> 25.6 us; 701x333 FP32, 7 shots, 17.1 -> 4.2 us.  What bounds the first:
+// VALU issue.  Per launch of 8 steps the 26,880 plain blocks issue 200 M wave
+// instructions, 14.5 a node and step, 781 k of the 759 k cycles of 332 us at 4 a
+// SIMD; the 6,976 slab blocks 135 M, 527 k of 602 k cycles.  Memory is behind
+// that: 1.32 GB past L2 at 4.0 TB/s, 0.46 GB at 1.9 TB/s.  44 % of a 64-row
+// tile's nodes are its rings.
 //
 // The arithmetic of a node is the single-step kernel's, operation for
 // operation (-ffp-contract=off), so the results equal n single-step launches
