@@ -207,8 +207,9 @@ int awcpml_get_two_step_align(const awcpml_plan *plan, int *enable);
 /* Time `nlaunches` two-step stencil launches alone (no source or receiver
  * work), in milliseconds; fails unless awcpml_set_time_block asked for two
  * steps and two-step launches apply.  2D: the same 2 * nlaunches steps in
- * launches of up to eight, as awcpml_advance makes them.  The state advances without sources; call awcpml_reset afterwards.  Measurement
- * support, no reference counterpart. */
+ * launches of up to eight, as awcpml_advance makes them.  The state advances
+ * without sources; call awcpml_reset afterwards.  Measurement support, no
+ * reference counterpart. */
 int awcpml_time_stencil2(awcpml_plan *plan, int nlaunches, double *ms_total);
 
 /* Force the kernels' 64-bit address offsets on any grid (enable != 0),
